@@ -167,8 +167,8 @@ int ns_int4_linear(void* out, const void* x, int64_t x_stride_row,
  * the device, each walking K = 4864).  Same operands, epilogues and RMSNorm
  * as ns_int4_linear; the fp32 partial sums of each split go to `workspace`
  * and the last split of a tile adds them in split order (deterministic) and
- * runs the epilogue.  The split count (up to 4) keeps tiles x splits within
- * 256 workgroups up to 128 tokens (register-dequant kernel); above (tiled
+ * runs the epilogue.  Up to 128 tokens the split count (up to 8) depends on
+ * how many workgroups the layer's tiles make; above (tiled
  * GEMM), the tiles of the last dispatch round split (all tiles when one round
  * holds them) when they fill at most half of the device's slots, within
  * those slots and with at least 8 K steps of 64 a split, so it depends on N,

@@ -25,6 +25,13 @@
 // matching 8 x values per step for each column tile.  The result D[n][m]
 // lands as four consecutive features of one token per lane: one 8-byte store.
 #include <algorithm>
+#ifdef NS_TUNE
+#include <cstdlib>
+#include <cstdio>
+#define NS_MINK (getenv("NS_K")?0:1024)
+#else
+#define NS_MINK 1024
+#endif
 
 #include "ns_common.h"
 
@@ -74,6 +81,9 @@ struct Int4LinearParams {
   // gemm_gh = group_size / 32, computed as umulhi(n, gemm_ghinv) (ceil(2^32 /
   // gemm_gh); exact since n * gemm_gh < 2^32) or n itself when gemm_gh is 1.
   uint32_t gemm_gh, gemm_ghinv;
+  // Group of a 128-wide chunk c: c / stream_cg with stream_cg = group_size /
+  // 128, the same way.
+  uint32_t stream_cg, stream_cginv;
 };
 
 // Device-scope (sc1) buffer accesses carry partials between workgroups, which
@@ -711,6 +721,458 @@ hipError_t launch_int4_linear(const Int4LinearParams& p, hipStream_t stream, int
   return hipLaunchKernel(fn, grid, dim3(64 * sh.waves), args, 0, stream);
 }
 
+// --------------------------------------------------------------------------
+// Long K at decode batch sizes: the weight stream.
+//
+// int4_linear_kernel gives each 16-feature tile a workgroup of its own whose
+// lanes load straight into the MFMA operand layout: neighbouring lanes hold
+// different rows, so each of their loads is up to 64 separate L1 accesses
+// (counted: 22 million a call for N = 28672, K = 3584 at 16 tokens, at about
+// one a cycle and CU the whole of its 46 us), every tile fetches all of x
+// again, and thousands of tiles are many short workgroups in turn.  Here:
+//  - a workgroup owns FT feature tiles and 16·NT tokens, so that the grid is
+//    about one round; its waves split the chunks of its K range;
+//  - a wave brings its own operands into its own part of LDS by
+//    global_load_lds with lanes running along the rows (the codes of a tile's
+//    chunk are 16 runs of 64 bytes, x rows runs of 256), R (chunk, tile) units
+//    of codes and the next chunk's x ahead, with no barrier between waves;
+//    neighbouring waves take neighbouring chunks, so the two halves of a
+//    128-byte line are read at the same time (contiguous runs of chunks per
+//    wave fetched 82 MB from HBM instead of 55);
+//  - a chunk's x is read into registers once and used for all FT tiles, and
+//    every code is dequantised once for all the tokens;
+//  - scales and zero points, strided by a row's groups, come into LDS as a
+//    table once (columns along the lanes);
+//  - the waves' sums meet in LDS, where each wave adds up and finishes its
+//    share of the 16x16 tiles of the result.
+// Dequantisation (21 VALU operations per 8 codes, dequant8_pairs) and the
+// stream then take about as long as each other; the rest is the launch, the
+// first loads and the reduction.  MI355X, graph-replayed, weights from HBM, us
+// before -> now at 1 / 16 / 32 / 64 / 128 tokens: 28672 x 3584 36.9 / 46 / 84 /
+// 163 / 244 -> 19.5 / 19.7 / 22.4 / 40 / 76; 3584 x 14336 18.5 / 26.4 / 46.7 /
+// 88.6 / 135 -> 14.6 / 14.9 / 16.7 / 24 / 37; 896 x 4864 6.9 / 7.5 / 8.4 /
+// 9.6 / 18.2 -> 6.4 / 6.6 / 6.7 / 7.3 / 8.8.
+// --------------------------------------------------------------------------
+
+// Eight codes -> weights in the order k = 0, 4, 1, 5, 2, 6, 3, 7, by the
+// arithmetic of dequant8_mix.  Nibbles e and e + 4 lie 16 bits apart, so one
+// and-or makes an f16 pair of them: 1024 + q for even e, 1024 + 16 q for odd
+// e (the nibble one position up), which one packed f16 add of -(1024 + z), or
+// one packed fma with 1/16 and -(64 + z), turns into q - z exactly.
+template <class DT>
+__device__ __forceinline__ typename DT::vec8 dequant8_pairs(uint32_t word, uint32_t zb, uint32_t zb16, float scale,
+                                                            uint32_t magic) {
+  typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+  constexpr uint32_t k16th = 0x2C002C00u;  // the f16 pair (1/16, 1/16)
+  typename DT::vec8 a;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t w = i < 2 ? word : word >> 8;
+    const uint32_t t = (w & (i & 1 ? 0x00F000F0u : 0x000F000Fu)) | magic;
+    const half2_t h = __builtin_bit_cast(half2_t, t);
+    const half2_t d = i & 1 ? __builtin_elementwise_fma(h, __builtin_bit_cast(half2_t, k16th),
+                                                        __builtin_bit_cast(half2_t, zb16))
+                            : h + __builtin_bit_cast(half2_t, zb);
+    const uint32_t u = __builtin_bit_cast(uint32_t, d);
+    float lo, up;
+    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(u), "v"(scale));
+    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(up) : "v"(u), "v"(scale));
+    a[2 * i] = static_cast<typename DT::T>(lo);
+    a[2 * i + 1] = static_cast<typename DT::T>(up);
+  }
+  return a;
+}
+__device__ __forceinline__ uint32_t zero_bias16_f16x2(uint32_t zb) {  // -(1024 + z) -> -(64 + z)
+  typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, zb) + half2_t{960, 960});
+}
+
+// Eight x values in the same order.
+template <class DT>
+__device__ __forceinline__ typename DT::vec8 pair_order(typename DT::vec8 v) {
+  const u32x4 d = __builtin_bit_cast(u32x4, v);
+  u32x4 o;
+  o[0] = __builtin_amdgcn_perm(d[2], d[0], 0x05040100u);
+  o[1] = __builtin_amdgcn_perm(d[2], d[0], 0x07060302u);
+  o[2] = __builtin_amdgcn_perm(d[3], d[1], 0x05040100u);
+  o[3] = __builtin_amdgcn_perm(d[3], d[1], 0x07060302u);
+  return __builtin_bit_cast(typename DT::vec8, o);
+}
+
+// LDS of one workgroup: per wave an x buffer (16·NT rows of one 128-wide
+// chunk) and a ring of R code slots (one tile's chunk, 1 KiB, each), then
+// the scales and zero-point words of up to kStreamCols groups per feature row.
+constexpr int kStreamCols = 32;
+template <int NT, int FT, int WAVES, int R>
+struct StreamCfg {
+  static constexpr int X_B = NT * 4096;
+  static constexpr int WAVE_B = X_B + R * 1024;
+  static constexpr int DM = R < 2 * FT ? 2 : 3;  // chunks before the last whose loads and waits differ
+  static constexpr int ROWS = FT * 16;
+  static constexpr int SC_B = ROWS * kStreamCols * 4;
+  static constexpr int ZP_B = ROWS * 16 * 4;
+  static constexpr int RED_B = WAVES * FT * NT * 1024;
+  static constexpr int STREAM_B = WAVES * WAVE_B + SC_B + ZP_B;
+  static constexpr int LDS = STREAM_B > RED_B ? STREAM_B : RED_B;
+  static_assert(R >= FT && R < DM * FT && R <= 16, "the waits below count on it");
+  static_assert(LDS <= 160 * 1024 - 64, "one workgroup fits a CU");
+};
+
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <int N>
+struct Int {
+  static constexpr int value = N;
+};
+
+template <class DT, int NT, int FT, int WAVES, int R>
+__global__ __launch_bounds__(WAVES * 64, WAVES / 4) void int4_stream_kernel(Int4LinearParams p) {
+  using C = StreamCfg<NT, FT, WAVES, R>;
+  constexpr int ESZ = sizeof(typename DT::T);
+  constexpr int TILES = FT * NT;  // 16x16 tiles of the result
+  constexpr int XD = 4 * NT;      // loads of a chunk's x
+  using V8 = typename DT::vec8;
+  using V4 = typename DT::vec4;
+  using T = typename DT::T;
+  __shared__ __attribute__((aligned(1024))) char smem[C::LDS];
+  const int lane = threadIdx.x & 63, row = lane & 15, grp = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int n0 = blockIdx.x * 16 * FT, m0 = blockIdx.y * 16 * NT;
+  const int S = static_cast<int>(gridDim.z), z = static_cast<int>(blockIdx.z);
+  const int chunks = p.K / 128;
+  const int cz0 = (chunks * z) / S, cz1 = (chunks * (z + 1)) / S;
+
+  char* const xbuf = smem + wave * C::WAVE_B;
+  char* const ring = xbuf + C::X_B;
+  char* const sc = smem + WAVES * C::WAVE_B;
+  char* const zp = sc + C::SC_B;
+
+  // Loader roles.  x: load d brings rows 4d .. 4d+3, 16-byte unit u of row r
+  // at LDS unit u ^ r, so that an operand read (16 rows, one unit) meets every
+  // bank once.  Codes: a tile's chunk is 16 rows of 64 bytes, piece q of row r
+  // at q ^ (r >> 2).  Rows past M repeat the last one and are never stored.
+  uint32_t xoff[XD];
+#pragma unroll
+  for (int d = 0; d < XD; ++d) {
+    const int r = 4 * d + (lane >> 4);
+    xoff[d] = static_cast<uint32_t>((static_cast<int64_t>(min(m0 + r, p.M - 1)) * p.x_stride + 8 * ((lane & 15) ^ (r & 15))) * ESZ);
+  }
+  const uint32_t coff = static_cast<uint32_t>(lane >> 2) * static_cast<uint32_t>(p.K / 2) +
+                        16u * ((lane & 3) ^ ((lane >> 4) & 3));
+  const uint32_t cread = 64 * row + 16 * (grp ^ ((row >> 2) & 3));
+  const int last_tile = p.N - 16;  // tiles past N repeat the last one and are not stored
+
+  floatx4 acc[FT][NT];
+#pragma unroll
+  for (int f = 0; f < FT; ++f)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[f][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t magic = f16_magic_pair();
+
+  // Group of chunk c (a chunk lies inside one group).
+  auto group_of = [&](int c) -> int {
+    return p.stream_cg == 1 ? c : static_cast<int>(__umulhi(static_cast<uint32_t>(c), p.stream_cginv));
+  };
+  // The zero-point byte of group g of a row lies in word (z3 + g - g0) / 4 of
+  // the row's words from group g0 on; z3 is the same for every tile (16 rows
+  // of any number of groups are whole words).
+  const uint32_t zrow = static_cast<uint32_t>(row) * static_cast<uint32_t>(p.groups);
+
+  for (int ph = cz0; ph < cz1; ph += kStreamCols) {
+    // Chunks ph .. pe-1; this wave takes ph + wave, + WAVES, ... (neighbouring
+    // waves read the two halves of a 128-byte line of codes at the same time).
+    const int pe = min(cz1, ph + kStreamCols);
+    const int n = (pe - ph - wave + WAVES - 1) / WAVES, U = n * FT;  // chunks and (chunk, tile) units
+    const int g0 = group_of(ph), gcols = group_of(pe - 1) - g0 + 1;
+    if (ph != cz0) __syncthreads();  // the tables of the last phase are read
+
+    // Tables: column c of row r at c ^ (r >> 1 & 7); zero-point word w at w ^ (r >> 2 & 3).
+    for (int d = wave; d < C::ROWS / 2; d += WAVES) {
+      const int r = 2 * d + (lane >> 5), c = min((lane & 31) ^ ((r >> 1) & 7), gcols - 1);
+      const uint32_t o = static_cast<uint32_t>(min(n0 + r, p.N - 1)) * static_cast<uint32_t>(p.groups) + g0 + c;
+      dma_lds4_off(p.scales, 4 * o, sc + d * 256);
+    }
+    for (int d = wave; d < C::ROWS / 4; d += WAVES) {
+      const int r = 4 * d + (lane >> 4), w = (lane & 15) ^ ((r >> 2) & 3);
+      const uint32_t o = static_cast<uint32_t>(min(n0 + r, p.N - 1)) * static_cast<uint32_t>(p.groups) + g0;
+      dma_lds4_off(p.zeros, min((o & ~3u) + 4 * w, (o + gcols - 1) & ~3u), zp + d * 256);
+    }
+
+    auto load_x = [&](int i) {
+      const char* base = p.x + static_cast<int64_t>(ph + wave + i * WAVES) * (128 * ESZ);
+#pragma unroll
+      for (int d = 0; d < XD; ++d) dma_lds16_off(base, xoff[d], xbuf + d * 1024);
+    };
+    // Units (chunk i, tile f) run through the ring's slots in order.
+    const uint8_t* const wbase = p.qweight + 64 * (ph + wave);
+    auto load_w = [&](int i, int f, int slot) {
+      const int nt = min(n0 + 16 * f, last_tile);
+      dma_lds16_off(wbase + static_cast<int64_t>(nt) * (p.K / 2) + 64 * WAVES * i, coff, ring + slot * 1024);
+    };
+
+    if (n > 0) {
+      load_x(0);
+#pragma unroll
+      for (int u = 0; u < R; ++u)
+        if (u < U) load_w(u / FT, u % FT, u);
+      // The tables and chunk 0's x have landed.
+      if (U >= R) wait_vm<R>();
+      else wait_vm<FT>();
+    } else {
+      wait_vm<0>();
+    }
+    __syncthreads();  // every wave's share of the tables
+
+    u32x4 codes, ncodes;
+    uint32_t scw, zpw, nscw, nzpw;
+    int slot = 0;  // of the unit read last
+    auto read_unit = [&](int i, int f, u32x4& cd, uint32_t& s_, uint32_t& z_) {
+      const int gi = group_of(ph + wave + i * WAVES) - g0;
+      const int w = (((zrow + g0) & 3u) + gi) >> 2;
+      cd = ds_read_b128(ring + slot * 1024 + cread);
+      s_ = ds_read_b32(sc + 4 * (row * kStreamCols + (gi ^ ((row >> 1) & 7))) + f * (64 * kStreamCols));
+      z_ = ds_read_b32(zp + 4 * (row * 16 + (w ^ ((row >> 2) & 3))) + f * 1024);
+    };
+    // One chunk, DIST chunks before the wave's last (at most DM: then any
+    // number).  With it known, so is how many of the wave's loads are younger
+    // than the one waited for, and what there is left to load.
+    auto chunk = [&](auto dist, int i) {
+      constexpr int DIST = decltype(dist)::value;
+      constexpr bool X_AHEAD = DIST >= 1;
+      if (i > 0) {  // younger than this chunk's x: the codes fetched during the last chunk
+        constexpr int k = (DIST + 2) * FT - R - 1;
+        wait_vm<(k < 0 ? 0 : k < FT ? k : FT)>();
+      }
+      V8 b[4][NT];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          b[j][t] = __builtin_bit_cast(V8, ds_read_b128(xbuf + t * 4096 + row * 256 + (((4 * grp + j) ^ row) << 4)));
+      lds_wait_all();
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) lds_ready(b[j][t]);
+      if constexpr (X_AHEAD) load_x(i + 1);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) b[j][t] = pair_order<DT>(b[j][t]);
+      const uint32_t zsh = 8 * ((zrow + group_of(ph + wave + i * WAVES)) & 3u);
+#pragma unroll
+      for (int f = 0; f < FT; ++f) {
+        constexpr int LEFT = (DIST + 1) * FT;  // units from this chunk's first on
+        const bool more = f + 1 < LEFT;
+        if (more) {
+          // The next unit's codes have landed; younger: the units after it up
+          // to R - 1, and the x fetched by this chunk.
+          constexpr int XA = X_AHEAD ? XD : 0;
+          switch (f + 2 + R - 1 <= LEFT ? R - 1 : LEFT - 2 - f) {
+#define NS_W(n) case n: wait_vm<(n) + XA>(); break;
+            NS_W(0) NS_W(1) NS_W(2) NS_W(3) NS_W(4) NS_W(5) NS_W(6) NS_W(7) NS_W(8) NS_W(9) NS_W(10) NS_W(11)
+            NS_W(12) NS_W(13) NS_W(14) NS_W(15)
+#undef NS_W
+            default: wait_vm<0>();
+          }
+          slot = slot + 1 == R ? 0 : slot + 1;
+          read_unit(f + 1 < FT ? i : i + 1, f + 1 < FT ? f + 1 : 0, ncodes, nscw, nzpw);
+        }
+        const uint32_t zb = zero_bias_f16x2((zpw >> zsh) & 0xFFu), zb16 = zero_bias16_f16x2(zb);
+        const float scale = __builtin_bit_cast(float, scw);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const V8 a = dequant8_pairs<DT>(codes[j], zb, zb16, scale, magic);
+#pragma unroll
+          for (int t = 0; t < NT; ++t) acc[f][t] = mfma16x16x32(DT{}, a, b[j][t], acc[f][t]);
+        }
+        if (more) {
+          lds_wait_all();
+          lds_ready(ncodes), lds_ready(nscw), lds_ready(nzpw);
+          if (f + 1 + R < LEFT) load_w(i + (f + 1 + R) / FT, (f + 1 + R) % FT, slot);  // into the slot just read
+          codes = ncodes;
+          scw = nscw;
+          zpw = nzpw;
+        }
+      }
+    };
+
+    if (n > 0) {
+      // Unit 0's codes: the other units of the prologue are younger.
+      if (U >= R) wait_vm<R - 1>();
+      else wait_vm<FT - 1>();
+      read_unit(0, 0, codes, scw, zpw);
+      lds_wait_all();
+      lds_ready(codes), lds_ready(scw), lds_ready(zpw);
+      if (R < U) load_w(R / FT, R % FT, 0);
+      for (int i = 0; i + C::DM < n; ++i) chunk(Int<C::DM>{}, i);
+      if constexpr (C::DM == 3)
+        if (n >= 3) chunk(Int<2>{}, n - 3);
+      if (n >= 2) chunk(Int<1>{}, n - 2);
+      chunk(Int<0>{}, n - 1);
+    }
+  }
+
+  // The waves' partial sums meet in LDS; wave w finishes tiles w, w + WAVES, ...
+  __syncthreads();
+  floatx4* const red = reinterpret_cast<floatx4*>(smem);
+#pragma unroll
+  for (int f = 0; f < FT; ++f)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) red[(wave * TILES + f * NT + t) * 64 + lane] = acc[f][t];
+  __syncthreads();
+  constexpr int OWN = (TILES + WAVES - 1) / WAVES;
+  floatx4 y4[OWN];
+#pragma unroll
+  for (int o = 0; o < OWN; ++o) {
+    const int i = wave + o * WAVES;
+    y4[o] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (i < TILES) {
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) y4[o] += red[(w * TILES + i) * 64 + lane];
+    }
+  }
+
+  if (S > 1) {
+    // Publish, count the arrival; the last split adds all S partials in split
+    // order (as int4_linear_kernel).
+    __shared__ unsigned last_arrival;
+    const int wg = static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x);
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(p.part, static_cast<short>(0), p.part_bytes, kBufferWord3);
+    auto off = [&](int zz, int i) { return (((wg * S + zz) * TILES + i) * 64 + lane) * 16; };
+#pragma unroll
+    for (int o = 0; o < OWN; ++o)
+      if (wave + o * WAVES < TILES)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, y4[o]), rs, off(z, wave + o * WAVES), 0, kSc1);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the partial stores are acknowledged
+    __syncthreads();                     // ... by every wave
+    if (threadIdx.x == 0)
+      last_arrival = __hip_atomic_fetch_add(&p.counters[wg], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                     static_cast<unsigned>(S - 1);
+    __syncthreads();
+    if (!last_arrival) return;
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+      if (wave + o * WAVES >= TILES) break;
+      y4[o] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int zz = 0; zz < S; ++zz)
+        y4[o] += __builtin_bit_cast(
+            floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, off(zz, wave + o * WAVES), 0, kSc1));
+    }
+    if (threadIdx.x == 0) __hip_atomic_store(&p.counters[wg], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+
+  // Features nf .. nf+3 of token m, rounded where the reference's separate
+  // tensor ops round.
+#pragma unroll
+  for (int o = 0; o < OWN; ++o) {
+    const int i = wave + o * WAVES;
+    if (i >= TILES) break;
+    const int nf = n0 + 16 * (i / NT) + 4 * grp, m = m0 + 16 * (i % NT) + row;
+    if (nf >= p.N || m >= p.M) continue;
+    float y[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float bias = p.bias ? from_model<DT>(static_cast<const T*>(p.bias)[nf + r]) : 0.f;
+      y[r] = from_model<DT>(to_model<DT>(y4[o][r] + bias));
+    }
+    if (p.epilogue == NS_EPILOGUE_SILU_MUL) {
+      T* dst = static_cast<T*>(p.out) + static_cast<int64_t>(m) * (p.N / 2) + nf / 2;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        dst[h] = to_model<DT>(from_model<DT>(to_model<DT>(silu_f32(y[2 * h]))) * y[2 * h + 1]);
+      continue;
+    }
+    V4 v;
+    if (p.epilogue == NS_EPILOGUE_RESIDUAL) {
+      const V4 res = *reinterpret_cast<const V4*>(static_cast<const T*>(p.residual) + static_cast<int64_t>(m) * p.N + nf);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = to_model<DT>(y[r] + from_model<DT>(res[r]));
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = to_model<DT>(y[r]);
+    }
+    *reinterpret_cast<V4*>(static_cast<T*>(p.out) + static_cast<int64_t>(m) * p.N + nf) = v;
+  }
+}
+
+struct StreamShape {
+  int nt, ft, waves, mtiles, gx, splits;
+};
+
+// Whether the stream kernel takes the call: more chunks than the one-chunk
+// kernels hold, whole 128-wide chunks and each inside one group.
+constexpr int kCUs = 256;
+bool stream_takes(int K, int group_size) { return K > NS_MINK && K % 128 == 0 && group_size % 128 == 0; }
+
+// Instantiated shapes: (NT, FT, WAVES, R).
+#define NS_INT4_STREAM_SHAPES(X) \
+  X(1, 1, 8, 2) X(1, 2, 8, 4) X(1, 3, 8, 5) X(1, 4, 8, 7) X(1, 5, 8, 9) X(1, 6, 8, 11) X(1, 7, 8, 12) X(1, 8, 8, 12) \
+  X(2, 1, 8, 2) X(2, 2, 8, 4) X(2, 3, 8, 5) X(2, 4, 8, 7) X(2, 5, 8, 9) X(2, 6, 8, 9) X(2, 7, 8, 9)
+
+// Token tile, feature tiles per workgroup and K splits by a cost in us fitted
+// to MI355X timings of K = 3584 and 14336 (bf16) and K = 4864 (fp16) layers at
+// 1 to 128 tokens: the KiB of codes that the busiest CU streams at 18 KiB/us
+// and of x (from L2) at 100, 0.2 per feature tile (its share of the
+// reduction), 1 per dispatch round, 0.4 per split (partials to publish and
+// add), and 0.7 plus a tenth of the stream for 32-token tiles.  At 16 tokens,
+// N = 28672, K = 3584 takes 19.7 us with 7 feature tiles (256 workgroups),
+// 20.5 with 8, 23.6 with 4 and 22.2 with 2; N = 3584, K = 14336 14.9 with 4
+// tiles and 4 splits, 17.4 with 1 and no split; N = 896, K = 4864 7.3 / 6.8 /
+// 6.8 / 7.1 with 1 tile and 1 / 2 / 3 / 4 splits.
+StreamShape stream_shape(int64_t M, int N, int K, bool can_split) {
+  const int tiles = N / 16, chunks = K / 128;
+  StreamShape best{};
+  float best_cost = 0.f;
+  for (int nt = 1; nt <= (M > 16 ? 2 : 1); ++nt) {
+    const int mtiles = static_cast<int>((M + 16 * nt - 1) / (16 * nt));
+    for (int ft = 1; ft <= 9 - nt; ++ft) {
+      const int gx = (tiles + ft - 1) / ft, wgs = gx * mtiles;
+      // (the arrival counters of a split call are limited, and filled CUs gain nothing from splits)
+      const int most = can_split && wgs < kCUs ? std::min(std::min(2 * kCUs / wgs, 8), chunks / 4) : 1;
+      for (int s = 1; s <= std::max(most, 1); ++s) {
+        const int rounds = (wgs * s + kCUs - 1) / kCUs;
+        const float kib = static_cast<float>(rounds * ft * ((chunks + s - 1) / s));
+        const float x_kib = kib / ft * (4 * nt);
+        const float cost = kib * (nt == 1 ? 1.f / 18 : 1.1f / 18) + x_kib * 0.01f + 0.2f * ft + rounds +
+                           (s > 1 ? 0.4f * s : 0.f) + 0.7f * (nt - 1);
+        if (best.ft == 0 || cost < best_cost) {
+          best = {nt, ft, 8, mtiles, gx, s};
+          best_cost = cost;
+        }
+      }
+    }
+  }
+#ifdef NS_TUNE
+  if (getenv("NS_FT")) best.ft = atoi(getenv("NS_FT"));
+  if (getenv("NS_W")) best.waves = atoi(getenv("NS_W"));
+  if (getenv("NS_X")) best.nt = atoi(getenv("NS_X"));
+  if (getenv("NS_S")) best.splits = can_split ? atoi(getenv("NS_S")) : 1;
+  best.mtiles = static_cast<int>((M + 16 * best.nt - 1) / (16 * best.nt));
+  best.gx = (tiles + best.ft - 1) / best.ft;
+  if (getenv("NS_V")) printf("M%d N%d K%d -> nt%d ft%d s%d wgs%d\n",(int)M,N,K,best.nt,best.ft,best.splits,best.gx*best.mtiles*best.splits);
+#endif
+  return best;
+}
+
+template <class DT>
+hipError_t launch_int4_stream(const Int4LinearParams& p, const StreamShape& s, hipStream_t stream) {
+  void* args[] = {const_cast<Int4LinearParams*>(&p)};
+  const void* fn = nullptr;
+#define NS_PICK(NT_, FT_, W_, R_)                  \
+  if (s.nt == NT_ && s.ft == FT_ && s.waves == W_) \
+    fn = reinterpret_cast<const void*>(&int4_stream_kernel<DT, NT_, FT_, W_, R_>);
+  NS_INT4_STREAM_SHAPES(NS_PICK)
+#undef NS_PICK
+  if (!fn) return hipErrorInvalidValue;
+  const dim3 grid(static_cast<unsigned>(s.gx), static_cast<unsigned>(s.mtiles), static_cast<unsigned>(s.splits));
+  return hipLaunchKernel(fn, grid, dim3(64 * s.waves), args, 0, stream);
+}
+
 bool aligned(const void* q, uintptr_t a) { return reinterpret_cast<uintptr_t>(q) % a == 0; }
 
 // --------------------------------------------------------------------------
@@ -779,11 +1241,6 @@ struct Cfg {
 // start of the workspace).
 constexpr int kMaxSplitTiles = 256;
 }  // namespace gemm
-
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 template <class DT, int BM, int BN, int NST, int WN>
 __global__ __launch_bounds__(gemm::THREADS, 2) void int4_gemm_kernel(Int4LinearParams p) {
@@ -1162,7 +1619,7 @@ struct SplitkLayout {
 // Token counts above kGemmMinRows take the GEMM (when K is a whole number of
 // its steps), the rest the fused kernel with 16 bytes of partials per lane,
 // tile and split.
-SplitkLayout splitk_layout(int64_t M, int N, int K) {
+SplitkLayout splitk_layout(int64_t M, int N, int K, bool stream) {
   SplitkLayout l{1, 0, 0};
   if (M <= 0) return l;
   if (M > kGemmMinRows) {
@@ -1171,6 +1628,10 @@ SplitkLayout splitk_layout(int64_t M, int N, int K) {
       l.splits = gs.splits;
       l.part_bytes = gemm_part_bytes(gs);
     }
+  } else if (stream) {
+    const StreamShape ss = stream_shape(M, N, K, true);
+    l.splits = ss.splits;
+    l.part_bytes = l.splits > 1 ? static_cast<int64_t>(ss.gx) * ss.ft * ss.mtiles * l.splits * ss.nt * 64 * 16 : 0;
   } else {
     const int mt = M <= 64 ? 16 : 64;
     const int64_t tiles = static_cast<int64_t>(N / 16) * ((M + mt - 1) / mt);
@@ -1181,6 +1642,18 @@ SplitkLayout splitk_layout(int64_t M, int N, int K) {
   return l;
 }
 static_assert(kSplitkCounterBytes % 256 == 0, "partials stay 256-byte aligned");
+
+// Workspace of a call: the group size decides between the kernels for up to
+// kGemmMinRows rows, so enough for either.
+size_t splitk_bytes(int64_t M, int N, int K) {
+  const SplitkLayout l = splitk_layout(M, N, K, false);
+  int64_t bytes = l.counter_bytes + l.part_bytes;
+  if (M <= kGemmMinRows && stream_takes(K, 128)) {
+    const SplitkLayout ls = splitk_layout(M, N, K, true);
+    bytes = std::max(bytes, ls.counter_bytes + ls.part_bytes);
+  }
+  return static_cast<size_t>(bytes);
+}
 
 int int4_linear_entry(void* out, const void* x, int64_t x_stride_row, const void* qweight, const void* scales,
                       const void* zeros, const void* bias, const void* residual, int epilogue,
@@ -1229,13 +1702,15 @@ int int4_linear_entry(void* out, const void* x, int64_t x_stride_row, const void
   // A 64-wide K step of the GEMM lies inside one group.
   const bool use_gemm = M > kGemmMinRows && !norm_weight && K % gemm::BK == 0 && group_size % gemm::BK == 0 &&
                         (!bias || aligned(bias, 8)) && aligned(zeros, 4) && small;
+  const bool use_stream = M <= kGemmMinRows && !norm_weight && stream_takes(K, group_size) && aligned(zeros, 4) && small;
   int splits = 1;
   if (splitk && (use_gemm || M <= kGemmMinRows)) {
-    const SplitkLayout l = splitk_layout(M, N, K);
-    if (l.splits > 1) {
-      if (!workspace || !aligned(workspace, 256) ||
-          workspace_bytes < static_cast<size_t>(l.counter_bytes + l.part_bytes) || l.part_bytes > 0x7FFFFFFF)
-        return NS_ERR_INVALID_ARG;
+    const bool have = workspace && aligned(workspace, 256) && workspace_bytes >= splitk_bytes(M, N, K);
+    // A call whose plain kernel splits needs the workspace; the weight stream
+    // runs unsplit without one.
+    if (splitk_layout(M, N, K, false).splits > 1 && !have) return NS_ERR_INVALID_ARG;
+    const SplitkLayout l = splitk_layout(M, N, K, use_stream);
+    if (l.splits > 1 && have && l.part_bytes <= 0x7FFFFFFF) {
       p.counters = static_cast<unsigned*>(workspace);
       p.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + l.counter_bytes);
       p.part_bytes = static_cast<int>(l.part_bytes);
@@ -1253,6 +1728,12 @@ int int4_linear_entry(void* out, const void* x, int64_t x_stride_row, const void
     p.gemm_gh = static_cast<uint32_t>(group_size / 32);
     p.gemm_ghinv = p.gemm_gh == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + p.gemm_gh - 1) / p.gemm_gh);
     e = dtype == NS_DTYPE_F16 ? launch_int4_gemm<F16>(p, gs, s) : launch_int4_gemm<BF16>(p, gs, s);
+  } else if (use_stream) {
+    const StreamShape ss = stream_shape(M, N, K, splits > 1);
+    p.stream_cg = static_cast<uint32_t>(group_size / 128);
+    p.stream_cginv =
+        p.stream_cg == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + p.stream_cg - 1) / p.stream_cg);
+    e = dtype == NS_DTYPE_F16 ? launch_int4_stream<F16>(p, ss, s) : launch_int4_stream<BF16>(p, ss, s);
   } else
     e = dtype == NS_DTYPE_F16 ? launch_int4_linear<F16>(p, s, splits) : launch_int4_linear<BF16>(p, s, splits);
   return e == hipSuccess ? NS_OK : NS_ERR_HIP;
@@ -1271,8 +1752,7 @@ extern "C" int ns_int4_linear(void* out, const void* x, int64_t x_stride_row,
 
 extern "C" size_t ns_int4_linear_splitk_workspace_size(int64_t M, int N, int K) {
   if (M < 0 || N <= 0 || K <= 0) return 0;
-  const ns::SplitkLayout l = ns::splitk_layout(M, N, K);
-  return static_cast<size_t>(l.counter_bytes + l.part_bytes);
+  return ns::splitk_bytes(M, N, K);
 }
 
 extern "C" int ns_int4_linear_splitk(void* out, const void* x, int64_t x_stride_row,

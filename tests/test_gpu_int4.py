@@ -585,3 +585,46 @@ def test_tiled_gemm_splits_the_last_rounds_tiles(dtype, N, K, M, epi):
     for t, what in ((first, "split"), (plain, "unsplit")):
         err = np.abs(t.double().cpu().numpy() - want)
         assert (err <= tol).all(), f"{what}: max err {err.max():.3e}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N,K,gs", [(16, 1152, 128), (80, 1280, 256), (112, 4224, 128), (4592, 1152, 384),
+                                    (4624, 1536, 128)],
+                         ids=lambda v: str(v))
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 128])
+def test_long_k_weight_stream(dtype, N, K, gs, M):
+    """Decode-size calls on K > 1024 layers against the oracle: one and many feature
+    tiles (a last workgroup with fewer tiles than the others), 9 to 33 chunks (one
+    more than a scale table holds, and fewer than the waves after a split), groups of
+    one, two and three chunks, part-filled token tiles, strided x rows; and the split
+    call (which rounds its partial sums in another order) within the same bound,
+    with its counters back at zero."""
+    from nanoserve_amd.quant import splitk_workspace_bytes
+
+    print(f"stream M={M} N={N} K={K} gs={gs} {dtype}", flush=True)
+    packed, s, z = (t.to(DEV) for t in _weights(N, K, gs, N + K))
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K + 8, generator=g).to(dtype)[:, :K]
+    res = torch.randn(M, N, generator=g).to(dtype)
+    b = (torch.randn(N, generator=g) * 0.1).to(dtype)
+    xd = torch.empty(M, K + 8, dtype=dtype, device=DEV)[:, :K].copy_(x)
+    ws = torch.zeros(max(splitk_workspace_bytes(N, K), 256), dtype=torch.uint8, device=DEV)
+    whole = int4_linear(xd, packed, s, z, b.to(DEV), gs, residual=res.to(DEV), method="fused")
+    split = int4_linear(xd, packed, s, z, b.to(DEV), gs, residual=res.to(DEV), method="fused", workspace=ws)
+    act = int4_linear(xd, packed, s, z, None, gs, silu_mul=True, method="fused", workspace=ws)
+    torch.cuda.synchronize()
+    assert not ws[:SPLITK_COUNTER_BYTES].any()
+    w = dequantize_int4_ref(packed.cpu().numpy(), s.cpu().numpy(), z.cpu().numpy(), gs, NAME[dtype])
+    y = int4_linear_ref(x.float().numpy(), w, b.float().numpy())
+    want = _round(y, dtype) + res.double().numpy()
+    tol = 2 * RTOL[dtype] * (np.abs(y) + np.abs(res.double().numpy())) + 1e-5 * max(1.0, np.abs(y).max())
+    for got, what in ((whole, "whole"), (split, "split")):
+        err = np.abs(got.double().cpu().numpy() - want)
+        assert (err <= tol).all(), f"{what}: max err {err.max():.3e}"
+    y = int4_linear_ref(x.float().numpy(), w, None)
+    gv, uv = _round(y[:, 0::2], dtype), _round(y[:, 1::2], dtype)
+    a = _round(gv / (1.0 + np.exp(-gv)), dtype)
+    # gate and up may each round the other way (one unit), then act and the product round.
+    tol = 4 * RTOL[dtype] * np.abs(a * uv) + 4 * RTOL[dtype] * np.abs(a * uv).max() * 1e-2 + 1e-4
+    err = np.abs(act.double().cpu().numpy() - _round(a * uv, dtype))
+    assert (err <= tol).all(), f"silu: max err {err.max():.3e}"
