@@ -25,13 +25,6 @@
 // matching 8 x values per step for each column tile.  The result D[n][m]
 // lands as four consecutive features of one token per lane: one 8-byte store.
 #include <algorithm>
-#ifdef NS_TUNE
-#include <cstdlib>
-#include <cstdio>
-#define NS_MINK (getenv("NS_K")?0:1024)
-#else
-#define NS_MINK 1024
-#endif
 
 #include "ns_common.h"
 
@@ -1107,7 +1100,7 @@ struct StreamShape {
 // Whether the stream kernel takes the call: more chunks than the one-chunk
 // kernels hold, whole 128-wide chunks and each inside one group.
 constexpr int kCUs = 256;
-bool stream_takes(int K, int group_size) { return K > NS_MINK && K % 128 == 0 && group_size % 128 == 0; }
+bool stream_takes(int K, int group_size) { return K > 1024 && K % 128 == 0 && group_size % 128 == 0; }
 
 // Instantiated shapes: (NT, FT, WAVES, R).
 #define NS_INT4_STREAM_SHAPES(X) \
@@ -1147,15 +1140,6 @@ StreamShape stream_shape(int64_t M, int N, int K, bool can_split) {
       }
     }
   }
-#ifdef NS_TUNE
-  if (getenv("NS_FT")) best.ft = atoi(getenv("NS_FT"));
-  if (getenv("NS_W")) best.waves = atoi(getenv("NS_W"));
-  if (getenv("NS_X")) best.nt = atoi(getenv("NS_X"));
-  if (getenv("NS_S")) best.splits = can_split ? atoi(getenv("NS_S")) : 1;
-  best.mtiles = static_cast<int>((M + 16 * best.nt - 1) / (16 * best.nt));
-  best.gx = (tiles + best.ft - 1) / best.ft;
-  if (getenv("NS_V")) printf("M%d N%d K%d -> nt%d ft%d s%d wgs%d\n",(int)M,N,K,best.nt,best.ft,best.splits,best.gx*best.mtiles*best.splits);
-#endif
   return best;
 }
 

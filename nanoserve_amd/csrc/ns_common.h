@@ -174,6 +174,31 @@ __device__ __forceinline__ uint32_t ds_read_b32(const void* lds) {
   asm volatile("ds_read_b32 %0, %1" : "=v"(r) : "v"(a));
   return r;
 }
+// The same reads at a byte address plus a constant offset (the instruction's
+// own), so that reads a constant apart share one address register.
+__device__ __forceinline__ uint32_t lds_addr(const void* lds) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) char*)(lds)));
+}
+template <int OFF>
+__device__ __forceinline__ u32x4 ds_read_b128_at(uint32_t a) {
+  static_assert(OFF >= 0 && OFF < 65536, "16-bit offset");
+  u32x4 r;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(a), "n"(OFF));
+  return r;
+}
+template <int OFF>
+__device__ __forceinline__ u32x2 ds_read_tr16_b64_at(uint32_t a) {
+  static_assert(OFF >= 0 && OFF < 65536, "16-bit offset");
+  u32x2 r;
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(a), "n"(OFF));
+  return r;
+}
+// Until at most N of the wave's LDS operations are pending (they complete in
+// order; other users of the counter only make it wait longer).
+template <int N>
+__device__ __forceinline__ void lds_wait() {
+  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
+}
 __device__ __forceinline__ void lds_wait_all() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 // Orders every later use of x after the preceding lds_wait_all().
 template <class V>

@@ -76,14 +76,9 @@ struct AttnParams {
 // slot_base | pair_base << 16, then its query length.  The decode kernel takes
 // the 200-byte base alone, so its launches do not carry the 3 KB schedule.
 struct PrefillParams : AttnParams {
+  int wide;  // host only: PrefillCfg's WIDE
   uint32_t plan[kPlanMax];
 };
-
-typedef short short4_t __attribute__((ext_vector_type(4)));
-
-// Address-space views for global_load_lds (global source, LDS destination).
-typedef __attribute__((address_space(1))) void* gbl_void_ptr;
-typedef __attribute__((address_space(3))) void* lds_void_ptr;
 
 // LDS swizzles of K and V tiles ([keys][D] rows of 16-byte units): unit c of
 // key k is stored at unit c ^ k_swz(k) (K) or c ^ v_swz(k) (V) of its row, so
@@ -818,34 +813,50 @@ __global__ __launch_bounds__(W * 64) void paged_decode_kernel(AttnParams p) {
 // from position 0 to the causal limit of its last column, KT keys per step.
 //
 // The workgroup is KG key groups of WC waves.  Wave i of every group owns the
-// same CT 16-column tiles; group k takes steps k, k + KG, k + 2KG, ... with
-// its own running (max, sum, O) and the groups are merged through LDS at the
-// end, so the dependent chain of steps is KG times shorter and each SIMD
-// holds KG waves.  Each step's K and V tiles go from HBM straight into LDS
+// same CT 16-column tiles; group k takes steps k, k + KG, ... with its own
+// running (max, sum, O), and the groups are merged through LDS at the end.
+// Each macro-step's (KG steps') K and V tiles go from HBM straight into LDS
 // with global_load_lds (16 bytes per lane, no registers), two macro-steps
-// (KG steps each) ahead of the one being computed, through a ring of three
-// macro-slots; every byte is read once per workgroup and one barrier per
-// macro-step hands a slot over.  The block-table entries of the keys come
-// first into LDS (a window of TBL entries), so the loads need no table round
-// trip of their own.
+// ahead of the one being computed, through a ring of three macro-slots; every
+// byte is read once per workgroup and one barrier per macro-step hands a slot
+// over.  The block-table entries of the keys come first into LDS (a window of
+// TBL entries), so the loads need no table round trip of their own.
 //
-// LDS layout of a stage: K tile then V tile, both [KT][D] rows of 16-byte
-// chunks, chunk c of key k stored at chunk c ^ k_swz(k) (K) or c ^ v_swz(k)
+// Two widths.  The narrow one (128 columns, two key groups of four waves, 32
+// columns a wave) halves the chain of steps and makes the most workgroups; the
+// wide one (384 columns at D = 64, 256 at D = 128, eight waves side by side)
+// loads each K/V tile for three / two times as many columns, and its waves
+// share one tile instead of two.  What bounds both is the vector ALU's issue
+// slots (SQ counters, 2048 rows x 7 heads behind 9392 keys, D = 64: 180 VALU
+// operations, 32 exponentials of four slots and 36 MFMAs per wave and 64 keys
+// x 32 columns, 1376 of about 1620 cycles in the wide kernel; 228 before the
+// operand reads took constant offsets and the table look-ups moved off the
+// loads' path) plus the barriers.  The host takes the wide one where it makes
+// enough workgroups (prefill_wide).
+//
+// LDS layout of a slot: K tile then V tile, both [KT][D] rows of 16-byte
+// chunks, chunk c of key k stored at chunk c ^ k_swz(k) (K) or c ^ pf_v_swz(k)
 // (V) of its row.  A DMA lane picks the global chunk that belongs at its LDS
 // slot, so the swizzle costs nothing on the write side and spreads the MFMA
 // operand reads (16-byte K rows; 8-byte transposing V reads) over all banks.
 // --------------------------------------------------------------------------
-template <int D, int CT_>
+
+// The transposing reads are served 32 lanes at a time, 8 keys of two
+// neighbouring chunks each; a row of D = 64 is half of the banks, so keys of
+// one parity share a half.
+template <int D>
+__device__ __forceinline__ int pf_v_swz(int key) {
+  return D == 64 ? ((key >> 1) & 3) << 1 : (key & 7) << 1;
+}
+
+template <int D, bool WIDE>
 struct PrefillCfg {
-  // Four key groups of two column waves (32 keys a step, 64 columns per
-  // workgroup) measured slower at c3 than two groups of four (51.0 against
-  // 45.2 us per call): twice the workgroups, still one per CU.
-  static constexpr int KG = 2;                  // key groups
-  static constexpr int WC = 4;                  // column waves per group
+  static constexpr int KG = WIDE ? 1 : 2;       // key groups
+  static constexpr int WC = WIDE ? 8 : 4;       // column waves per group
   static constexpr int W = KG * WC;             // waves per workgroup
   static constexpr int THREADS = W * 64;
-  static constexpr int CT = CT_;                // 16-column tiles per wave
-  static constexpr int KT = D == 64 ? 64 : 32;  // keys per step (8 KiB per tile)
+  static constexpr int CT = WIDE && D == 64 ? 3 : 2;       // 16-column tiles per wave (registers: two waves per SIMD)
+  static constexpr int KT = WIDE || D == 64 ? 64 : 32;     // keys per step
   static constexpr int NT = KT / 16, NC = D / 32, NN = D / 16;
   static constexpr int CPR = D / 8;             // 16-byte chunks per key row
   static constexpr int TILE = KT * D * 2;       // bytes of one K or V tile
@@ -859,10 +870,22 @@ struct PrefillCfg {
   static constexpr int PU = CT * (NN + 1);      // 16-byte units per lane of a split's partial
   static constexpr int SLOT_BYTES = WC * PU * 64 * 16;
   static_assert(DMA >= 1 && DMA * THREADS * 16 == KG * TILE && TILE % 1024 == 0, "loads must tile a macro-step");
-  static_assert(NT % 2 == 0, "P^T operand pairs two 16-key tiles");
-  static_assert(WC * NF * 64 * 4 <= RING, "merge buffer fits the ring");
+  static_assert(KG == 1 || WC * NF * 64 * 4 <= RING, "merge buffer fits the ring");
 };
 
+// f(constant 0), ..., f(constant N - 1).
+template <int V>
+struct Const {
+  static constexpr int value = V;
+  __device__ constexpr operator int() const { return V; }
+};
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(Const<I>{});
+    static_for<N, I + 1>(f);
+  }
+}
 
 // Wait until at most N of this wave's vector-memory operations are pending,
 // drain its LDS operations, then barrier.  Written as one asm statement so the
@@ -875,13 +898,13 @@ __device__ __forceinline__ void stage_barrier() {
 
 constexpr int kPrefillThreads = 512;
 
-template <class DT, int D, int CT, class BTI>
+template <class DT, int D, bool WIDE, class BTI>
 __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(PrefillParams p) {
-  using Cfg = PrefillCfg<D, CT>;
+  using Cfg = PrefillCfg<D, WIDE>;
   static_assert(Cfg::THREADS == kPrefillThreads, "launch bounds match the workgroup");
   using T = typename DT::T;
   using V8 = typename DT::vec8;
-  constexpr int KT = Cfg::KT, NT = Cfg::NT, NC = Cfg::NC, NN = Cfg::NN, KG = Cfg::KG;
+  constexpr int CT = Cfg::CT, KT = Cfg::KT, NT = Cfg::NT, NC = Cfg::NC, NN = Cfg::NN, KG = Cfg::KG;
   constexpr int CPR = Cfg::CPR, TILE = Cfg::TILE, DMA = Cfg::DMA, W = Cfg::W;
   __shared__ __attribute__((aligned(16))) char smem[Cfg::LDS];
   int* tbl = reinterpret_cast<int*>(smem + Cfg::RING);
@@ -919,12 +942,14 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(PrefillP
   int64_t L64 = load_index(p.seq_lens, s, p.sl64);
   if (ql64 <= 0 || (p.skip_decode_rows && ql64 == 1)) return;
   if (q0 < 0 || q0 + ql64 > p.num_tokens) return;
-  const int64_t ncols = ql64 * G;
-  const int64_t ncb = (ncols + Cfg::COLS - 1) / Cfg::COLS;
-  int64_t cb = blockIdx.x;
+  // Columns are int32: 2^31 of them would be a query of more than 256 GiB.
+  const uint32_t Gu = static_cast<uint32_t>(G);
+  const int ncols = static_cast<int>(ql64 * G);
+  const int ncb = static_cast<int>((static_cast<uint32_t>(ncols) + Cfg::COLS - 1) / Cfg::COLS);
+  int cb = static_cast<int>(blockIdx.x);
   bool plan_broken = false;
   if (p.plan_n > 0) {
-    const int64_t rcb = blockIdx.x / Hkv / nsplit;
+    const int rcb = static_cast<int>(blockIdx.x / static_cast<uint32_t>(Hkv) / static_cast<uint32_t>(nsplit));
     if (rcb >= ncb) return;
     cb = ncb - 1 - rcb;
     // A device query length the host plan did not describe is a broken
@@ -936,8 +961,8 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(PrefillP
       nsplit = 1;
     }
   }
-  const int64_t c_wg = cb * Cfg::COLS;
-  if (c_wg >= ncols) return;
+  if (cb >= ncb) return;
+  const int c_wg = cb * Cfg::COLS;
   L64 = L64 < p.max_ctx ? L64 : p.max_ctx;
   const int L = static_cast<int>(L64 > 0 ? L64 : 0);
   const int64_t ctx0 = L - ql64;  // absolute position of query row 0 (may be negative)
@@ -945,39 +970,40 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(PrefillP
   const int bs_mask = (1 << bs_shift) - 1;
 
   // Keys the workgroup needs: up to the causal limit of its last column.
-  const int64_t c_last_wg = (ncols < c_wg + Cfg::COLS ? ncols : c_wg + Cfg::COLS) - 1;
-  int64_t kv_end64 = ctx0 + c_last_wg / G + 1;
+  auto last_row = [&](int c0, int n) {  // query row of the last of up to n columns from c0 on
+    return static_cast<int64_t>(static_cast<uint32_t>((ncols - c0 < n ? ncols : c0 + n) - 1) / Gu);
+  };
+  int64_t kv_end64 = ctx0 + last_row(c_wg, Cfg::COLS) + 1;
   kv_end64 = kv_end64 < L ? kv_end64 : L;
   const int kv_end = static_cast<int>(kv_end64 > 0 ? kv_end64 : 0);
 
   // This wave's columns: Q^T operands, causal limits, output rows.
-  const int64_t c_wave = c_wg + wc * CT * 16;
+  const int c_wave = c_wg + wc * CT * 16;
   const bool wave_on = c_wave < ncols;
   int kv_end_w = 0;
   int64_t qmin_w = -1;
   if (wave_on) {
-    const int64_t c_last = (ncols < c_wave + CT * 16 ? ncols : c_wave + CT * 16) - 1;
-    const int64_t e = ctx0 + c_last / G + 1;
+    const int64_t e = ctx0 + last_row(c_wave, CT * 16) + 1;
     kv_end_w = static_cast<int>(e < 0 ? 0 : (e < L ? e : L));
-    qmin_w = ctx0 + c_wave / G;
+    qmin_w = ctx0 + static_cast<uint32_t>(c_wave) / Gu;
   }
   V8 qop[CT][NC];
   int lim[CT];  // last key position a column may see (-1: none)
-  int64_t orow[CT];
-  bool cval[CT];
+  // Element offset of a column's query and output row.
+  auto row_of = [&](int c) {
+    const uint32_t qi = static_cast<uint32_t>(c) / Gu, h = static_cast<uint32_t>(c) - qi * Gu;
+    return ((q0 + qi) * p.num_heads + static_cast<int64_t>(kvh) * G + h) * D;
+  };
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
-    const int64_t c = c_wave + ct * 16 + c16;
-    cval[ct] = c < ncols;
-    const int64_t qi = cval[ct] ? c / G : 0;
-    const int64_t h = cval[ct] ? c - qi * G : 0;
-    const int64_t qpos = ctx0 + qi;
-    lim[ct] = cval[ct] ? static_cast<int>(qpos < kv_end_w - 1 ? qpos : kv_end_w - 1) : -1;
-    orow[ct] = ((q0 + qi) * p.num_heads + static_cast<int64_t>(kvh) * G + h) * D;
-    const T* qrow = reinterpret_cast<const T*>(p.query) + orow[ct];
+    const int c = c_wave + ct * 16 + c16;
+    const bool cval = c < ncols;
+    const int64_t qpos = ctx0 + (cval ? static_cast<uint32_t>(c) / Gu : 0);
+    lim[ct] = cval ? static_cast<int>(qpos < kv_end_w - 1 ? qpos : kv_end_w - 1) : -1;
+    const T* qrow = reinterpret_cast<const T*>(p.query) + row_of(cval ? c : 0);
 #pragma unroll
     for (int c2 = 0; c2 < NC; ++c2) {
-      qop[ct][c2] = cval[ct] ? load16<DT>(qrow + 32 * c2 + 8 * g) : zero8<DT>();
+      qop[ct][c2] = cval ? load16<DT>(qrow + 32 * c2 + 8 * g) : zero8<DT>();
       // A negative scale moves into Q (exact sign flips), so the softmax can
       // take maxima over raw scores and fold the scale into one FMA.
       if (p.scale_log2 < 0.f)
@@ -1015,78 +1041,121 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(PrefillP
   int e0 = 0;      // first table entry of the current window
   int kv_win = 0;  // keys covered by the window's entries (and below kv_end)
 
-  // Start the K/V loads of macro-step M into macro-slot `slot` (stages
-  // slot * KG + k, k < KG, one per step).  Load u of wave w covers the 1 KiB
-  // piece b = u * W + w of the macro-step's K (and of its V): piece b % PT of
-  // step M * KG + b / PT, lane `lane` filling its 16-byte slot b % PT * 64 +
-  // lane.  Keys past the window or kv_end read an in-bounds slot; their
-  // scores are masked and their V values replaced by zero when read.
-  auto dma_macro = [&](int M, int slot) {
-    constexpr int PT = TILE / 1024;  // 1 KiB pieces per tile
+  // K/V loads of macro-step M (one step per key group): load u of wave w covers
+  // the 1 KiB piece b = u * W + w of its K (and of its V) tiles, piece b % PT of
+  // step M * KG + b / PT, lane `lane` filling its 16-byte chunk.  The cache slot
+  // of a lane's key is looked up one macro-step before its loads are issued.
+  // Keys past the window or kv_end (and invalid blocks) take slot 0, in bounds;
+  // their scores are masked and their V values replaced by zero when read.
+  constexpr int PT = TILE / 1024;  // 1 KiB pieces per tile
+  auto slot_of = [&](int M, int u) -> uint32_t {
+    const int b = u * W + w, t = (M * KG + b / PT) * KT + (b % PT * 64 + lane) / CPR;
+    const bool in = t < kv_win;
+    const int blk = tbl[in ? (t >> bs_shift) - e0 : 0];
+    return in && blk >= 0 ? (static_cast<uint32_t>(blk) << bs_shift) + (t & bs_mask) : 0u;
+  };
+  const uint32_t row_bytes = static_cast<uint32_t>(slot_stride * sizeof(T));
+  auto dma = [&](int slot, const uint32_t (&cslot)[DMA]) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < DMA; ++u) {
-      const int b = u * W + w;
-      const int k = b / PT, piece = b % PT;
-      char* st = smem + (slot * KG + k) * 2 * TILE;
-      const int pos = piece * 64 + lane;
-      const int key = pos / CPR, pc = pos % CPR;
-      const int t = (M * KG + k) * KT + key;
-      const bool in = t < kv_win;
-      const int blk = tbl[in ? (t >> bs_shift) - e0 : 0];
-      const bool valid = in && blk >= 0;
-      const int64_t off = valid ? ((static_cast<int64_t>(blk) << bs_shift) + (t & bs_mask)) * slot_stride : 0;
-      const T* gk = kbase + off + ((pc ^ k_swz(key)) << 3);
-      const T* gv = vbase + off + ((pc ^ v_swz(key)) << 3);
-      __builtin_amdgcn_global_load_lds((gbl_void_ptr)(gk), (lds_void_ptr)(st + piece * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((gbl_void_ptr)(gv), (lds_void_ptr)(st + TILE + piece * 1024), 16, 0, 0);
+      const int b = u * W + w, pos = b % PT * 64 + lane, key = pos / CPR, pc = pos % CPR;
+      char* st = smem + (slot * KG + b / PT) * 2 * TILE + b % PT * 1024;
+      const uint64_t off = static_cast<uint64_t>(cslot[u]) * row_bytes;
+      dma_lds16(reinterpret_cast<const char*>(kbase) + off + ((pc ^ k_swz(key & 15)) << 4), st);
+      dma_lds16(reinterpret_cast<const char*>(vbase) + off + ((pc ^ pf_v_swz<D>(key & 15)) << 4), st + TILE);
     }
   };
+  // Operand addresses within a tile.  K: key 16j + c16, chunk 4 c2 + g.  V^T:
+  // k-slot 4h + e of lane group g is key 32pb + 16h + 4g + e, matching P^T;
+  // ds_read_b64_tr_b16 gives lane i of a 16-lane group element e = element i &
+  // 3 of the 8 bytes lane (i >> 2) + 4e of the group addressed, so lane c16 of
+  // group g points at head dims 16n + 4 (c16 & 3) .. +3 of key 32pb + 16h + 4g
+  // + (c16 >> 2) and receives V^T row 16n + c16 at keys 32pb + 16h + 4g +
+  // 0..3.  Both swizzles repeat every 16 keys, so j, pb and h are constants.
+  uint32_t koff[NC];
+#pragma unroll
+  for (int c2 = 0; c2 < NC; ++c2) koff[c2] = c16 * (D * 2) + (((4 * c2 + g) ^ k_swz(c16)) << 4);
+  const int vkey = 4 * g + (c16 >> 2);
+  const uint32_t voff = vkey * (D * 2) + ((((c16 & 3) >> 1) ^ pf_v_swz<D>(vkey)) << 4) + (c16 & 1) * 8;
 
-  // One step of this wave's columns from `stage`.
-  auto compute = [&](int stage, int step) {
+  // One step of this wave's columns from ring tile pair `slot`.
+  auto compute = [&](int slot, int step) __attribute__((always_inline)) {
     const int tb = step * KT;
     if (tb >= kv_end_w) return;
-    const char* kt = smem + stage * 2 * TILE;
-    const char* vt = kt + TILE;
+    // S^T = K Q^T, every K read issued first.  All the operand reads are asm:
+    // the compiler's wait-count pass would put an s_waitcnt vmcnt(0) in front
+    // of reads it cannot tell from the loads in flight into the ring.
     floatx4 sacc[CT][NT];
+    {
+      u32x4 kr[NT][NC];
+      const uint32_t base = lds_addr(smem + slot * 2 * TILE);
+      uint32_t at[NC];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const int key = 16 * j + c16;
-      V8 kop[NC];
+      for (int c2 = 0; c2 < NC; ++c2) at[c2] = base + koff[c2];
+      static_for<NT>([&](auto j) __attribute__((always_inline)) {
 #pragma unroll
-      for (int c2 = 0; c2 < NC; ++c2)
-        kop[c2] = *reinterpret_cast<const V8*>(kt + key * D * 2 + (((4 * c2 + g) ^ k_swz(key)) << 4));
+        for (int c2 = 0; c2 < NC; ++c2) kr[j][c2] = ds_read_b128_at<j * 16 * D * 2>(at[c2]);
+      });
+      static_for<NT>([&](auto j) __attribute__((always_inline)) {
+        lds_wait<(NT - 1 - j) * NC>();
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        sacc[ct][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int c2 = 0; c2 < NC; ++c2) lds_ready(kr[j][c2]);
 #pragma unroll
-        for (int c2 = 0; c2 < NC; ++c2) sacc[ct][j] = mfma16x16x32(DT{}, kop[c2], qop[ct][c2], sacc[ct][j]);
-      }
+        for (int c2 = 0; c2 < NC; ++c2)
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+            sacc[ct][j] = mfma16x16x32(DT{}, __builtin_bit_cast(V8, kr[j][c2]), qop[ct][c2],
+                                       c2 == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : sacc[ct][j]);
+      });
     }
-    // The V^T operands of the whole step (see the PV product below), issued
-    // now as asm so their LDS latency hides behind the softmax.  Through the
-    // builtin, the compiler's wait-count pass would put an s_waitcnt vmcnt(0)
-    // in front of the first one (it cannot tell them from the K/V loads in
-    // flight into the ring), draining the prefetch of the next macro-steps.
-    const int d0 = 4 * (c16 & 3);
-    u32x2 vraw[NT / 2][NN][2];
+    // V^T operands: of the whole step, or of 32 keys at a time where that is
+    // more than 32 registers, the first issued now so their LDS latency hides behind
+    // the softmax.
+    constexpr int VP = NT / 2 * NN <= 8 ? NT / 2 : 1;  // 32-key parts held at once
+    u32x2 vraw[VP][NN][2];
+    const uint32_t vbase_l = lds_addr(smem + slot * 2 * TILE + TILE);
+    auto read_v = [&](auto pb0) __attribute__((always_inline)) {
+      static_for<NN>([&](auto n) __attribute__((always_inline)) {
+        const uint32_t at = vbase_l + (voff ^ (n << 5));
+        static_for<VP>([&](auto i) __attribute__((always_inline)) {
+          vraw[i][n][0] = ds_read_tr16_b64_at<(pb0 + i) * 32 * D * 2>(at);
+          vraw[i][n][1] = ds_read_tr16_b64_at<(pb0 + i) * 32 * D * 2 + 16 * D * 2>(at);
+        });
+      });
+    };
+    V8 va[VP][NN];
+    const bool vfull = tb + KT <= kv_end;
+    auto take_v = [&](int pb0) __attribute__((always_inline)) {
+      lds_wait_all();
 #pragma unroll
-    for (int pb = 0; pb < NT / 2; ++pb)
+      for (int i = 0; i < VP; ++i)
 #pragma unroll
-      for (int n = 0; n < NN; ++n)
+        for (int n = 0; n < NN; ++n) {
+          lds_ready(vraw[i][n][0]);
+          lds_ready(vraw[i][n][1]);
+          va[i][n] = __builtin_bit_cast(
+              V8, u32x4{vraw[i][n][0][0], vraw[i][n][0][1], vraw[i][n][1][0], vraw[i][n][1][1]});
+          if (!vfull) {  // keys at or past kv_end (only in the last step) contribute zero
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int key = 32 * pb + 16 * h + 4 * g + (c16 >> 2);
-          const int d = 16 * n + d0;
-          vraw[pb][n][h] = ds_read_tr16_b64(vt + key * D * 2 + (((d >> 3) ^ v_swz(key)) << 4) + ((d & 7) << 1));
+            for (int e = 0; e < 8; ++e) {
+              const int key = 32 * (pb0 + i) + 16 * (e >> 2) + 4 * g + (e & 3);
+              va[i][n][e] = tb + key < kv_end ? va[i][n][e] : static_cast<T>(0.f);
+            }
+          }
         }
+    };
+    read_v(Const<0>{});
     // Online softmax in base 2 (sc = |scale| * log2 e).  When every key of the
     // step precedes every column of the wave, the maximum is taken over raw
     // scores and p = exp2(s * sc - m) is one FMA; otherwise key
     // tb + 16j + 4g + r of a column is masked by the column's limit.
     const bool full = tb + KT - 1 <= qmin_w;
-    const bool vfull = tb + KT <= kv_end;
-    V8 pt[CT][NT / 2], va[NT / 2][NN];
+    V8 pt[CT][NT / 2];
+    auto pv = [&](int ct, int pb, const V8 (&v)[NN]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int n = 0; n < NN; ++n) acc[ct][n] = mfma16x16x32(DT{}, v[n], pt[ct][pb], acc[ct][n]);
+      lacc[ct] = mfma16x16x32(DT{}, ones_row, pt[ct][pb], lacc[ct]);
+    };
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
       float sv[NT][4];
@@ -1138,38 +1207,20 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(PrefillP
           pt[ct][pb][4 + e] = static_cast<T>(sv[2 * pb + 1][e]);
         }
       // O^T += V^T P^T for this column tile, right after its softmax: the
-      // MFMAs run while the next tile's softmax issues.  k-slot 4h + e of lane
-      // group g is key 32pb + 16h + 4g + e, matching P^T.  ds_read_b64_tr_b16
-      // gives lane i of a 16-lane group element e = element i & 3 of the 8
-      // bytes lane (i >> 2) + 4e of the group addressed, so lane c16 of group
-      // g points at head dims 16n + 4 (c16 & 3) .. +3 of key 32pb + 16h + 4g +
-      // (c16 >> 2) and receives V^T row 16n + c16 at keys 32pb + 16h + 4g +
-      // 0..3.  Keys at or past kv_end (only in the last step) contribute zero.
-      if (ct == 0) {
-        lds_wait_all();
+      // MFMAs run while the next tile's softmax issues.
+      if constexpr (VP == NT / 2) {
+        if (ct == 0) take_v(0);
 #pragma unroll
-        for (int pb = 0; pb < NT / 2; ++pb)
-#pragma unroll
-          for (int n = 0; n < NN; ++n) {
-            lds_ready(vraw[pb][n][0]);
-            lds_ready(vraw[pb][n][1]);
-            va[pb][n] = __builtin_bit_cast(
-                V8, u32x4{vraw[pb][n][0][0], vraw[pb][n][0][1], vraw[pb][n][1][0], vraw[pb][n][1][1]});
-            if (!vfull) {
-#pragma unroll
-              for (int e = 0; e < 8; ++e) {
-                const int key = 32 * pb + 16 * (e >> 2) + 4 * g + (e & 3);
-                va[pb][n][e] = tb + key < kv_end ? va[pb][n][e] : static_cast<T>(0.f);
-              }
-            }
-          }
+        for (int pb = 0; pb < NT / 2; ++pb) pv(ct, pb, va[pb]);
       }
+    }
+    if constexpr (VP < NT / 2) {
+      static_for<NT / 2>([&](auto pb) __attribute__((always_inline)) {
+        take_v(pb);
+        if constexpr (pb + 1 < NT / 2) read_v(Const<pb + 1>{});
 #pragma unroll
-      for (int pb = 0; pb < NT / 2; ++pb) {
-#pragma unroll
-        for (int n = 0; n < NN; ++n) acc[ct][n] = mfma16x16x32(DT{}, va[pb][n], pt[ct][pb], acc[ct][n]);
-        lacc[ct] = mfma16x16x32(DT{}, ones_row, pt[ct][pb], lacc[ct]);
-      }
+        for (int ct = 0; ct < CT; ++ct) pv(ct, pb, va[0]);
+      });
     }
   };
 
@@ -1177,17 +1228,17 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(PrefillP
   // Macro-step M covers steps M * KG + k, k < KG (step M * KG + k by group k).
   // A split runs macro-steps [M_begin, M_end) of the column block's range.
   constexpr int MKEYS = KG * KT;
-  const int nmacro = (kv_end + MKEYS - 1) / MKEYS;
-  int nsplit_eff = 1, M_begin = 0, M_end = nmacro;
+  const int nsteps = (kv_end + MKEYS - 1) / MKEYS;
+  int nsplit_eff = 1, M_begin = 0, M_end = nsteps;
   if (nsplit > 1) {
-    nsplit_eff = nmacro > split_mk ? (nmacro + split_mk - 1) / split_mk : 1;
+    nsplit_eff = nsteps > split_mk ? (nsteps + split_mk - 1) / split_mk : 1;
     if (split >= nsplit_eff) return;  // no keys for this split: it does not arrive
     M_begin = split * split_mk;
-    M_end = M_begin + split_mk < nmacro ? M_begin + split_mk : nmacro;
+    M_end = M_begin + split_mk < nsteps ? M_begin + split_mk : nsteps;
   }
-  const int win_macro = (Cfg::TBL << bs_shift) / MKEYS;
-  for (int M0 = M_begin; M0 < M_end; M0 += win_macro) {
-    const int M1 = M0 + win_macro < M_end ? M0 + win_macro : M_end;
+  const int win_steps = (Cfg::TBL << bs_shift) / MKEYS;
+  for (int M0 = M_begin; M0 < M_end; M0 += win_steps) {
+    const int M1 = M0 + win_steps < M_end ? M0 + win_steps : M_end;
     e0 = (M0 * MKEYS) >> bs_shift;
     kv_win = M1 * MKEYS < kv_end ? M1 * MKEYS : kv_end;
     const int ne_all = ((kv_win + bs_mask) >> bs_shift) - e0;
@@ -1213,17 +1264,26 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(PrefillP
     }
     __syncthreads();
 
-    // Macro-steps M0 .. M1-1 through the three slots: at the top of macro-step
-    // M the loads of M+1 may still be in flight (2 * DMA per thread), M's
-    // have landed once every wave has waited for its own and passed the
-    // barrier; then M+2's loads go into the slot M-1 used.  Macro-steps past
-    // M1 still load (nothing valid) so the pending count stays exact.
-    dma_macro(M0, 0);
-    dma_macro(M0 + 1, 1);
+    // Macro-steps M0 .. M1-1 through the three slots: at the top of macro-step M the loads
+    // of M+1 may still be in flight (2 * DMA per thread), M's have landed once
+    // every wave has waited for its own and passed the barrier; then M+2's
+    // loads go into the slot M-1 used.  Steps past M1 still load (nothing
+    // valid) so the pending count stays exact.
+    uint32_t cslot[DMA];
+    auto look_up = [&](int step) __attribute__((always_inline)) {
+#pragma unroll
+      for (int u = 0; u < DMA; ++u) cslot[u] = slot_of(step, u);
+    };
+    look_up(M0);
+    dma(0, cslot);
+    look_up(M0 + 1);
+    dma(1, cslot);
+    look_up(M0 + 2);
     int slot = 0;
     for (int M = M0; M < M1; ++M) {
       stage_barrier<2 * DMA>();
-      dma_macro(M + 2, slot == 0 ? 2 : slot - 1);
+      dma(slot == 0 ? 2 : slot - 1, cslot);
+      look_up(M + 3);
       compute(slot * KG + kg, M * KG + kg);
       slot = slot == 2 ? 0 : slot + 1;
     }
@@ -1277,8 +1337,8 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(PrefillP
     // Split-K: park this split's state in its slot ([wave][float][lane], a
     // bad table entry as l = NaN), count the arrival, and let the last split
     // of the column block merge all slots in split order.
-    const int pair = pair_base + static_cast<int>(kvh * ncb + cb);
-    const int slot0 = slot_base + (kvh * static_cast<int>(ncb) + static_cast<int>(cb)) * nsplit;
+    const int pair = pair_base + kvh * ncb + cb;
+    const int slot0 = slot_base + (kvh * ncb + cb) * nsplit;
     const __amdgpu_buffer_rsrc_t pr =
         __builtin_amdgcn_make_buffer_rsrc(p.pf_part, static_cast<short>(0), p.pf_part_bytes, kBufferWord3);
     // Slot layout [wave][ct][unit][lane] of 16-byte units: unit 0 is
@@ -1363,9 +1423,10 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(PrefillP
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const float lsum = group4_sum_swap(l_run[ct]);
-    if (!cval[ct]) continue;
+    const int c = c_wave + ct * 16 + c16;
+    if (c >= ncols) continue;
     const float inv = bad_out ? NAN : (lsum > 0.f ? 1.f / lsum : 0.f);
-    T* orow_p = reinterpret_cast<T*>(p.out) + orow[ct];
+    T* orow_p = reinterpret_cast<T*>(p.out) + row_of(c);
 #pragma unroll
     for (int n = 0; n < NN; ++n) {
       typename DT::vec4 v4;
@@ -1379,9 +1440,6 @@ __global__ __launch_bounds__(kPrefillThreads) void paged_prefill_kernel(PrefillP
 // --------------------------------------------------------------------------
 // Host side.
 // --------------------------------------------------------------------------
-// 16-column tiles per prefill wave (columns per workgroup = 64 * kPrefillTiles).
-constexpr int kPrefillTiles = 2;
-
 // Decode launch shape: kDecodeWaves waves per workgroup, each with a ring of
 // decode_ring<D> chunk slots (16 KiB of LDS per wave at head_dim 64, 32 KiB
 // at 128).  Two chunks in flight per wave measured faster than three or
@@ -1409,12 +1467,9 @@ struct WorkspaceLayout {
 // block), and the bytes of one slot: a workgroup's per-lane softmax state.
 constexpr int kPrefillSlots = 512;
 size_t prefill_slot_bytes(int head_dim) {
-  return head_dim == 64 ? PrefillCfg<64, kPrefillTiles>::SLOT_BYTES : PrefillCfg<128, kPrefillTiles>::SLOT_BYTES;
+  return head_dim == 64 ? PrefillCfg<64, false>::SLOT_BYTES : PrefillCfg<128, false>::SLOT_BYTES;
 }
-constexpr size_t kPrefillRegion =
-    size_t{kPrefillSlots} * (PrefillCfg<64, kPrefillTiles>::SLOT_BYTES > PrefillCfg<128, kPrefillTiles>::SLOT_BYTES
-                                 ? PrefillCfg<64, kPrefillTiles>::SLOT_BYTES
-                                 : PrefillCfg<128, kPrefillTiles>::SLOT_BYTES);
+constexpr size_t kPrefillRegion = size_t{kPrefillSlots} * PrefillCfg<128, false>::SLOT_BYTES;
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
@@ -1579,24 +1634,27 @@ hipError_t launch_attention(AttnParams& p, PrefillParams& pp, const DecodePlanAr
   if (p.decode_only) return launch_decode_rows<DT, D>(p, build, decode_grid, stream);
 
   void* pargs[] = {&pp};
-  using PCfg = PrefillCfg<D, kPrefillTiles>;
-  const void* vk = pp.bt64 ? reinterpret_cast<const void*>(&paged_prefill_kernel<DT, D, kPrefillTiles, int64_t>)
-                           : reinterpret_cast<const void*>(&paged_prefill_kernel<DT, D, kPrefillTiles, int32_t>);
+  const int pf_cols = pp.wide ? PrefillCfg<D, true>::COLS : PrefillCfg<D, false>::COLS;
+  const void* vk =
+      pp.wide ? (pp.bt64 ? reinterpret_cast<const void*>(&paged_prefill_kernel<DT, D, true, int64_t>)
+                         : reinterpret_cast<const void*>(&paged_prefill_kernel<DT, D, true, int32_t>))
+              : (pp.bt64 ? reinterpret_cast<const void*>(&paged_prefill_kernel<DT, D, false, int64_t>)
+                         : reinterpret_cast<const void*>(&paged_prefill_kernel<DT, D, false, int32_t>));
   dim3 vgrid;
   if (pp.plan_n > 0) {
     vgrid = dim3(static_cast<unsigned>(pf_grid_x), static_cast<unsigned>(pp.plan_n), 1);
   } else {
     const int64_t cols = static_cast<int64_t>(max_query_len) * pp.group;
-    const int64_t nblk = (cols + PCfg::COLS - 1) / PCfg::COLS;
+    const int64_t nblk = (cols + pf_cols - 1) / pf_cols;
     if (nblk > 0x7FFFFFFF) return hipErrorInvalidValue;
     vgrid = dim3(static_cast<unsigned>(nblk), pp.num_kv_heads, num_seqs);
   }
-  if (!launch_decode) return hipLaunchKernel(vk, vgrid, dim3(PCfg::THREADS), pargs, 0, stream);
+  if (!launch_decode) return hipLaunchKernel(vk, vgrid, dim3(kPrefillThreads), pargs, 0, stream);
 
   if (!aux) {
     hipError_t e = launch_decode_rows<DT, D>(p, build, decode_grid, stream);
     if (e != hipSuccess) return e;
-    return hipLaunchKernel(vk, vgrid, dim3(PCfg::THREADS), pargs, 0, stream);
+    return hipLaunchKernel(vk, vgrid, dim3(kPrefillThreads), pargs, 0, stream);
   }
   hipError_t e = hipEventRecord(aux->fork, stream);
   if (e == hipSuccess) e = hipStreamWaitEvent(aux->stream, aux->fork, 0);
@@ -1605,7 +1663,7 @@ hipError_t launch_attention(AttnParams& p, PrefillParams& pp, const DecodePlanAr
   // else fails (an unjoined fork would also break a graph capture).
   const hipError_t ed = launch_decode_rows<DT, D>(p, build, decode_grid, aux->stream);
   const hipError_t er = hipEventRecord(aux->join, aux->stream);
-  const hipError_t ev = hipLaunchKernel(vk, vgrid, dim3(PCfg::THREADS), pargs, 0, stream);
+  const hipError_t ev = hipLaunchKernel(vk, vgrid, dim3(kPrefillThreads), pargs, 0, stream);
   const hipError_t ej = er == hipSuccess ? hipStreamWaitEvent(stream, aux->join, 0) : er;
   return ed != hipSuccess ? ed : (ev != hipSuccess ? ev : ej);
 }
@@ -1614,6 +1672,38 @@ bool aligned16(const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0;
 
 int64_t host_index(const void* a, int is64, int64_t i) {
   return is64 ? static_cast<const int64_t*>(a)[i] : static_cast<const int32_t*>(a)[i];
+}
+
+// Whether the batch's multi-row sequences take the wide prefill kernel: its
+// column blocks must fill the CUs, with the last round's loss small enough.
+// Graph-replayed on MI355X, us, narrow / wide (wide column blocks): D = 64
+// (14 / 2 heads, fp16) one prompt of 8192 tokens 219 / 271 (280), six of about
+// 1850 119 / 123 (412), eight 151 / 143 (546), one of 16000 695 / 628 (546).
+// D = 128 (28 / 4 heads, bf16) one prompt of 2600 112 / 118 (268), 3000 141.5
+// / 134 (308), 4000 213 / 176.5 (412), two of about 3700 421 / 337 (852), one
+// of 16000 2302 / 1810 (1636).  A single round does too at D = 128 if its
+// blocks are about as long as each other (the longest sets the span): two
+// chunks of 1024 behind up to 8000 keys 349 / 312 (224), against one prompt of
+// 2048, whose blocks grow from nothing, 76 / 96 (212).  Chunks that leave much
+// of a wide block empty keep the narrow one.
+bool prefill_wide(const void* lens, int lens64, const void* qsl, int qsl64, int num_seqs, int group, int num_kv_heads,
+                  int head_dim) {
+  const int64_t cols = head_dim == 64 ? PrefillCfg<64, true>::COLS : PrefillCfg<128, true>::COLS;
+  int64_t blocks = 0, used = 0;   // column blocks, and the columns in them
+  double total = 0, longest = 0;  // keys
+  for (int i = 0; i < num_seqs; ++i) {
+    const int64_t ql = host_index(qsl, qsl64, i + 1) - host_index(qsl, qsl64, i);
+    if (ql <= 1) continue;
+    const int64_t n = (ql * group + cols - 1) / cols * num_kv_heads;
+    const double L = static_cast<double>(host_index(lens, lens64, i));
+    blocks += n;
+    used += ql * group * num_kv_heads;
+    total += n * (L - 0.5 * ql);
+    longest = L > longest ? L : longest;
+  }
+  if (used < 0.6 * cols * blocks) return false;
+  if (head_dim == 64) return blocks >= 512;
+  return blocks >= 288 || (blocks >= 192 && total >= 0.6 * longest * blocks);
 }
 
 // Fill pp.plan with the prefill schedule from host query offsets and lengths:
@@ -1626,7 +1716,7 @@ int64_t host_index(const void* a, int is64, int64_t i) {
 // fit.  Returns the sequences listed (0: no plan, the launch then uses the
 // full grid without splits) and the grid width.
 int build_prefill_plan(PrefillParams& pp, const void* lens, int lens64, const void* qsl, int qsl64, int num_seqs,
-                       int cols_per_wg, int macro_keys, int& grid_x) {
+                       int cols_per_wg, int macro_keys, int max_slots, int& grid_x) {
   constexpr int kCUs = 256, kMinSplitMacro = 4, kMaxListed = kPlanMax / 3;
   struct Seq {
     int s, ncb;
@@ -1675,7 +1765,7 @@ int build_prefill_plan(PrefillParams& pp, const void* lens, int lens64, const vo
       }
       const int64_t items = static_cast<int64_t>(pp.num_kv_heads) * q.ncb * nsplit;
       if (nsplit > 1) {
-        if (slots + items > kPrefillSlots || slots > 0xFFFF || pairs > 0xFFFF) {
+        if (slots + items > max_slots || slots > 0xFFFF || pairs > 0xFFFF) {
           fits = false;
           break;
         }
@@ -1979,12 +2069,20 @@ int paged_attention_entry(void* out, const void* query, const void* k_cache, con
   if (!is_decode_only) {
     static_cast<AttnParams&>(pp) = p;
     pp.plan_n = 0;
+    pp.wide = 0;
     if (seq_lens_host && qsl_host) {
-      const int mkeys = head_dim == 64 ? PrefillCfg<64, kPrefillTiles>::KG * PrefillCfg<64, kPrefillTiles>::KT
-                                       : PrefillCfg<128, kPrefillTiles>::KG * PrefillCfg<128, kPrefillTiles>::KT;
+      pp.wide = prefill_wide(seq_lens_host, seq_lens_host_is_int64, qsl_host, query_start_loc_host_is_int64, num_seqs,
+                             group, num_kv_heads, head_dim);
+      const bool d64 = head_dim == 64;
+      const int cols = pp.wide ? (d64 ? PrefillCfg<64, true>::COLS : PrefillCfg<128, true>::COLS)
+                               : PrefillCfg<64, false>::COLS;
+      const int mkeys = pp.wide || !d64 ? 64 : 128;  // KG * KT
+      const size_t slot = !pp.wide ? prefill_slot_bytes(head_dim)
+                                   : (d64 ? PrefillCfg<64, true>::SLOT_BYTES : PrefillCfg<128, true>::SLOT_BYTES);
       pp.plan_n = build_prefill_plan(pp, seq_lens_host, seq_lens_host_is_int64, qsl_host,
-                                     query_start_loc_host_is_int64, num_seqs, PrefillCfg<64, kPrefillTiles>::COLS,
-                                     mkeys, pf_grid_x);
+                                     query_start_loc_host_is_int64, num_seqs, cols, mkeys,
+                                     static_cast<int>(wl.pf_part_bytes / slot), pf_grid_x);
+      if (!pp.plan_n) pp.wide = 0;
     }
   }
 

@@ -324,6 +324,27 @@ def test_prefill_block_size_one_crosses_table_windows(seqs, qls):
     _assert_close(_run(q, kc, vc, md, 0.125), paged_attention_ref(q, kc, vc, md, 0.125), torch.float16)
 
 
+@pytest.mark.parametrize("block_size", [1, 16])
+@pytest.mark.parametrize("D,cols,dtype", [(64, 384, torch.float16), (128, 256, torch.bfloat16)])
+def test_prefill_wide_column_blocks(D, cols, dtype, block_size):
+    """Batches with enough column blocks take the wide kernel (384 / 256 columns a
+    workgroup): at least 512 blocks over 8 KV heads of 16 query heads, chunks of one
+    row more and fewer than a block, of a few columns, of several blocks and of two
+    rows, contexts that end inside, at and just past a 64-key step, one past a
+    4096-entry table window (block size 1), and decode rows beside them."""
+    rows = cols // 16
+    qls = ([rows, rows - 1, rows + 1, 3 * rows] * 16)[:60] + [2, 5, 1, 1]
+    seqs = [q + c for q, c in zip(qls, [0, 64 - rows, 65, 300, 1] * 13)]
+    seqs[7] += 4096
+    q, kc, vc, md, _, _ = _case(seqs, qls, 128, 8, D, block_size, dtype)
+    scale = 1.0 / math.sqrt(D)
+    print(f"wide prefill D={D} bs={block_size}", flush=True)
+    _assert_close(_run(q, kc, vc, md, scale), paged_attention_ref(q, kc, vc, md, scale), dtype)
+    # Without host offsets the same call runs the narrow kernel over the full grid.
+    md.seq_lens_cpu = md.query_start_loc_cpu = None
+    _assert_close(_run(q, kc, vc, md, scale), paged_attention_ref(q, kc, vc, md, scale), dtype)
+
+
 @pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
 def test_prefill_long_context_splits_match_unsplit(D, dtype):
     """With host offsets the long key ranges of a chunked prefill are split
