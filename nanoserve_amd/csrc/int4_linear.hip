@@ -25,6 +25,7 @@
 // matching 8 x values per step for each column tile.  The result D[n][m]
 // lands as four consecutive features of one token per lane: one 8-byte store.
 #include <algorithm>
+#include <cmath>
 
 #include "ns_common.h"
 
@@ -816,11 +817,6 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int N>
-struct Int {
-  static constexpr int value = N;
-};
-
 template <class DT, int NT, int FT, int WAVES, int R>
 __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void int4_stream_kernel(Int4LinearParams p) {
   using C = StreamCfg<NT, FT, WAVES, R>;
@@ -1001,11 +997,11 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void int4_stream_kernel(Int4
       lds_wait_all();
       lds_ready(codes), lds_ready(scw), lds_ready(zpw);
       if (R < U) load_w(R / FT, R % FT, 0);
-      for (int i = 0; i + C::DM < n; ++i) chunk(Int<C::DM>{}, i);
+      for (int i = 0; i + C::DM < n; ++i) chunk(Const<C::DM>{}, i);
       if constexpr (C::DM == 3)
-        if (n >= 3) chunk(Int<2>{}, n - 3);
-      if (n >= 2) chunk(Int<1>{}, n - 2);
-      chunk(Int<0>{}, n - 1);
+        if (n >= 3) chunk(Const<2>{}, n - 3);
+      if (n >= 2) chunk(Const<1>{}, n - 2);
+      chunk(Const<0>{}, n - 1);
     }
   }
 
@@ -1249,13 +1245,19 @@ __global__ __launch_bounds__(gemm::THREADS, 2) void int4_gemm_kernel(Int4LinearP
   // tile b whole; the rest take split z of tile gemm_whole + st, unit
   // gemm_whole + z * split_tiles + st, so one round of splits covers every
   // split tile.  The dispatcher deals workgroup i to XCD i % 8; workgroup i
-  // takes unit b from a contiguous eighth of the units per XCD, so the
+  // takes unit b from a contiguous eighth of its kind of units per XCD, so the
   // workgroups of one XCD share x row blocks in that XCD's L2 (down_proj at
   // 1024 tokens 34.4 -> 32.7 us, o_proj at 2048 14.7 -> 13.7 us on MI355X).
+  // Whole tiles and splits are dealt apart: eighths of all the units gave one
+  // XCD every split and the others more whole tiles than they have slots for,
+  // a second full round (down_proj at 4700 tokens, 512 whole tiles of 128 x 64
+  // and 6 split 4 times: 107.3 -> 76.7 us).
   const int gx = p.gemm_gx;
-  const int b = [] {
-    const int units = gridDim.x, q = units >> 3, r = units & 7, xcd = blockIdx.x & 7;
-    return xcd * q + min(xcd, r) + static_cast<int>(blockIdx.x >> 3);
+  const int b = [&] {
+    const bool split = static_cast<int>(blockIdx.x) >= p.gemm_whole;
+    const int at = split ? p.gemm_whole : 0, units = split ? static_cast<int>(gridDim.x) - at : p.gemm_whole;
+    const int i = static_cast<int>(blockIdx.x) - at, q = units >> 3, r = units & 7, xcd = i & 7;
+    return at + xcd * q + min(xcd, r) + (i >> 3);
   }();
   const int split_tiles = ((p.M + BM - 1) / BM) * gx - p.gemm_whole;
   int S = 1, z = 0, st = 0, tile = b;
@@ -1308,12 +1310,10 @@ __global__ __launch_bounds__(gemm::THREADS, 2) void int4_gemm_kernel(Int4LinearP
       edst[j] = r * 4;
     }
   }
-  // This lane's operand rows: features WF wn + 16 fi + c16 of the tile; the
-  // zero-point byte of group gi sits at byte (zrow + gi) & 3 of its word.
-  uint32_t zrow[FT];
-#pragma unroll
-  for (int fi = 0; fi < FT; ++fi)
-    zrow[fi] = static_cast<uint32_t>(min(n0 + C::WF * wn + 16 * fi + c16, p.N - 1)) * static_cast<uint32_t>(p.groups);
+  // This lane's operand rows: features WF wn + 16 fi + c16 of the tile, 16
+  // rows apart (whole zero-point words), so the zero-point byte of group gi
+  // sits at byte (zrow + gi) & 3 of its word for each of them.
+  const uint32_t zrow = static_cast<uint32_t>(c16) * static_cast<uint32_t>(p.groups);
   auto group_of = [&](int n) -> int {
     return p.gemm_gh == 1 ? n : static_cast<int>(__umulhi(static_cast<uint32_t>(n), p.gemm_ghinv));
   };
@@ -1348,36 +1348,51 @@ __global__ __launch_bounds__(gemm::THREADS, 2) void int4_gemm_kernel(Int4LinearP
     else if (n == 1) wait_vm<C::PS>();
     else wait_vm<0>();
   };
-  // The A operands of step s: this lane's codes of rows WF wn + 16 fi + c16,
-  // k of the step in one group per lane, dequantised into both sub-steps.
-  auto dequant_step = [&](int s, V8 (&a)[FT][2]) {
+  // The A operands of a step: this lane's codes of rows WF wn + 16 fi + c16, k
+  // of the step in one group per lane, dequantised into both sub-steps; the B
+  // operands (x rows of this wave's tokens) of sub-step j.  All these reads are
+  // asm with explicit waits: left to the compiler, each B read was issued one
+  // or two MFMAs before its use and every pair of MFMAs waited for LDS.
+  struct Raw {
+    u32x2 words;
+    uint32_t scale, zword;
+  };
+  const uint32_t crow = 32 * (C::WF * wn + c16) + 16 * ((g >> 1) ^ ((c16 >> 3) & 1)) + 8 * (g & 1);
+  const uint32_t srow = 4 * (C::WF * wn + c16);
+  uint32_t brow[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) brow[j] = (C::WT * wm + c16) * ROW_B + (((2 * g + j) ^ ((c16 >> 1) & 7)) << 4);
+  auto read_raw = [&](int s, Raw (&raw)[FT]) {
     const int st = stage(s);
-    const uint32_t gi = static_cast<uint32_t>(group_of(2 * s));  // both halves of a step share a group
+    const uint32_t ca = lds_addr(cst(st)) + crow, sa = lds_addr(sst(st)) + srow, za = lds_addr(zst(st)) + srow;
+    static_for<FT>([&](auto fi) {
+      raw[fi].words = ds_read_b64_at<fi * 512>(ca);
+      raw[fi].scale = ds_read_b32_at<fi * 64>(sa);
+      raw[fi].zword = ds_read_b32_at<fi * 64>(za);
+    });
+  };
+  auto dequant_step = [&](int s, Raw (&raw)[FT], V8 (&a)[FT][2]) {
+    const uint32_t sh = 8 * ((zrow + static_cast<uint32_t>(group_of(2 * s))) & 3u);  // a step lies inside one group
 #pragma unroll
     for (int fi = 0; fi < FT; ++fi) {
-      const int r = C::WF * wn + 16 * fi + c16;
-      const u32x2 words =
-          *reinterpret_cast<const u32x2*>(cst(st) + 32 * r + 16 * ((g >> 1) ^ ((r >> 3) & 1)) + 8 * (g & 1));
-      const float scale = *reinterpret_cast<const float*>(sst(st) + 4 * r);
-      const uint32_t zword = *reinterpret_cast<const uint32_t*>(zst(st) + 4 * r);
-      const uint32_t zb = zero_bias_f16x2((zword >> (8 * ((zrow[fi] + gi) & 3u))) & 0xFFu);
-      a[fi][0] = dequant8_mix<DT>(words[0], zb, scale, magic);
-      a[fi][1] = dequant8_mix<DT>(words[1], zb, scale, magic);
+      lds_ready(raw[fi].words), lds_ready(raw[fi].scale), lds_ready(raw[fi].zword);
+      const float scale = __builtin_bit_cast(float, raw[fi].scale);
+      const uint32_t zb = zero_bias_f16x2((raw[fi].zword >> sh) & 0xFFu);
+      a[fi][0] = dequant8_mix<DT>(raw[fi].words[0], zb, scale, magic);
+      a[fi][1] = dequant8_mix<DT>(raw[fi].words[1], zb, scale, magic);
     }
   };
-  // The MFMAs of step s: A from registers, B (x rows of this wave's tokens)
-  // read from the step's stage as each token tile's turn comes.
-  auto mfma_step = [&](int s, const V8 (&a)[FT][2]) {
-    const char* xt = xst(stage(s));
+  auto read_b = [&](int s, int j, u32x4 (&b)[TT]) {
+    const uint32_t at = lds_addr(xst(stage(s))) + brow[j];
+    static_for<TT>([&](auto ti) { b[ti] = ds_read_b128_at<ti * 16 * ROW_B>(at); });
+  };
+  auto mfma_half = [&](int j, u32x4 (&b)[TT], const V8 (&a)[FT][2]) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int ti = 0; ti < TT; ++ti) {
+      lds_ready(b[ti]);
 #pragma unroll
-      for (int ti = 0; ti < TT; ++ti) {
-        const int row = C::WT * wm + 16 * ti + c16;
-        const V8 b = *reinterpret_cast<const V8*>(xt + row * ROW_B + (((2 * g + j) ^ ((row >> 1) & 7)) << 4));
-#pragma unroll
-        for (int fi = 0; fi < FT; ++fi) acc[fi][ti] = mfma16x16x32(DT{}, a[fi][j], b, acc[fi][ti]);
-      }
+      for (int fi = 0; fi < FT; ++fi)
+        acc[fi][ti] = mfma16x16x32(DT{}, a[fi][j], __builtin_bit_cast(V8, b[ti]), acc[fi][ti]);
     }
   };
 
@@ -1390,7 +1405,12 @@ __global__ __launch_bounds__(gemm::THREADS, 2) void int4_gemm_kernel(Int4LinearP
   wait_steps(min(s1 - 1 - s0, NST - 2));
   __syncthreads();
   V8 acur[FT][2];
-  dequant_step(s0, acur);
+  {
+    Raw raw[FT];
+    read_raw(s0, raw);
+    lds_wait_all();
+    dequant_step(s0, raw, acur);
+  }
   for (int s = s0; s < s1 - 1; ++s) {
     // Step s+1's loads have landed (those up to step s+NST-2 may fly); past
     // the barrier every wave is done with step s-1, whose stage takes step
@@ -1398,16 +1418,33 @@ __global__ __launch_bounds__(gemm::THREADS, 2) void int4_gemm_kernel(Int4LinearP
     wait_steps(min(s1 - 1, s + NST - 2) - (s + 1));
     __syncthreads();
     if (s + NST - 1 < s1) dma(s + NST - 1, stage(s + NST - 1));
+    Raw raw[FT];
+    u32x4 b0[TT], b1[TT];
+    read_raw(s + 1, raw);
+    read_b(s, 0, b0);
+    lds_wait<TT>();
     V8 anext[FT][2];
-    dequant_step(s + 1, anext);
-    mfma_step(s, acur);
+    dequant_step(s + 1, raw, anext);
+    read_b(s, 1, b1);
+    lds_wait<TT>();
+    mfma_half(0, b0, acur);
+    lds_wait_all();
+    mfma_half(1, b1, acur);
 #pragma unroll
     for (int fi = 0; fi < FT; ++fi) {
       acur[fi][0] = anext[fi][0];
       acur[fi][1] = anext[fi][1];
     }
   }
-  mfma_step(s1 - 1, acur);
+  {
+    u32x4 b0[TT], b1[TT];
+    read_b(s1 - 1, 0, b0);
+    read_b(s1 - 1, 1, b1);
+    lds_wait<TT>();
+    mfma_half(0, b0, acur);
+    lds_wait_all();
+    mfma_half(1, b1, acur);
+  }
 
   if (S > 1) {
     // Publish this split's sums, count the arrival; the last split of the
@@ -1429,15 +1466,26 @@ __global__ __launch_bounds__(gemm::THREADS, 2) void int4_gemm_kernel(Int4LinearP
                      static_cast<unsigned>(S - 1);
     __syncthreads();
     if (!last_arrival) return;
+    // Split by split, every tile's loads in flight at once (tile by tile, S
+    // loads one after the other, the merge was a chain of FT * TT * S trips to
+    // memory: down_proj at 1024 tokens, 56 tiles of 128 x 128 split 4 times,
+    // 44.9 -> 33.3 us).
 #pragma unroll
     for (int fi = 0; fi < FT; ++fi)
 #pragma unroll
-      for (int ti = 0; ti < TT; ++ti) {
-        floatx4 sum = {0.f, 0.f, 0.f, 0.f};
-        for (int zz = 0; zz < S; ++zz)
-          sum += __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, off(zz, fi, ti), 0, kSc1));
-        acc[fi][ti] = sum;
-      }
+      for (int ti = 0; ti < TT; ++ti) acc[fi][ti] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int zz = 0; zz < S; ++zz) {
+      floatx4 part[FT][TT];
+#pragma unroll
+      for (int fi = 0; fi < FT; ++fi)
+#pragma unroll
+        for (int ti = 0; ti < TT; ++ti)
+          part[fi][ti] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, off(zz, fi, ti), 0, kSc1));
+#pragma unroll
+      for (int fi = 0; fi < FT; ++fi)
+#pragma unroll
+        for (int ti = 0; ti < TT; ++ti) acc[fi][ti] += part[fi][ti];
+    }
     if (tid == 0) __hip_atomic_store(&p.counters[st], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
@@ -1501,38 +1549,71 @@ constexpr int gemm_lds(int bm, int bn, int nst) {
   return nst * (bm * gemm::ROW_B + bn * gemm::BK / 2 + 2 * bn * 4) + 16;
 }
 
-// Tile shape and split count of a GEMM call, from measurements on MI355X
-// (fp16, Qwen2.5-0.5B projections, graph-replayed).  128 x 128 tiles when
-// they still give two workgroups per CU (gate|up from 1024 tokens: 44.8 /
-// 66.3 us at 1024 / 2048 tokens against 46.9 / 86.7 with 64 x 128 tiles,
-// both unsplit);
-// 128-token x 64-feature tiles for long-K layers with enough of them
-// (down_proj at 2048 tokens, split twice: 49.1 us against 53.9 with 64 x 128
-// tiles); 64 x 64 tiles otherwise, the most workgroups for short calls (qkv /
-// o / down at 256 tokens: 10.4 / 10.8 / 21.6 us, against 13.8 / 14.8 / 30.7
-// with 64 x 128).  When the caller gave a workspace and the tiles of the last
-// dispatch round (all of them, if one round holds every tile) fill at most
-// half of the device's slots, those tiles split their K loop, at least 8
-// steps a split: shorter splits write and read back more fp32 partials than
-// the idle slots win (gate|up at 1024 / 2048 tokens, its last round's 128 x
-// 128 tiles split into 4-5 steps: 49.4 / 74.9 us against 39.5 / 64.9 unsplit).
+// Tile shape and split of a GEMM call: the cheapest by a model of the device.
+// A CU runs up to `slots` / 256 tiles of a shape at a time; a step of one costs
+// `alone` us, of k together alone + beside * (k - 1), since they share the CU's
+// matrix cores.  Full rounds run whole.  Of the last round's tiles, those past
+// the last multiple of a round, or of one tile per CU, may split their K loop,
+// when the caller gave a workspace and the splits fit the slots that are left:
+// at least 8 steps a split (shorter ones write and read back more fp32 partials
+// than the idle slots win: gate|up at 1024 / 2048 tokens, its last round's
+// tiles split into 4-5 steps, 49.4 / 74.9 us against 39.5 / 64.9 unsplit), and
+// 2.5 us + `merge` per split a CU for the partials.  A part-filled layer of
+// tiles counts 0.6 as a full one: its chain is what the call waits for.
+//
+// The constants fit 54 layers and token counts with every shape and split
+// forced (MI355X, fp16, graph-replayed; 129 to 10000 tokens, 896 x 896 to
+// 28672 x 3584): the pick is the fastest in 43, within 5% in 52 and 11% behind
+// in two (1536 x 1536 and 2304 x 1536 at 1024 tokens, 18.6 / 22.5 us against
+// 16.7 / 20.2).  Against shapes by thresholds on the tile count and splits of a
+// last round only, both measured: down_proj (896 x 4864) at 512 / 1500 / 4700
+// tokens 24.4 / 50.4 / 112 -> 20.5 / 31.4 / 73.7 us, 3584 x 14336 at 200 / 800
+// / 1200 / 2000 tokens 74.7 / 176 / 313 / 366 -> 55.1 / 144 / 209 / 288 us,
+// 28672 x 3584 at 200 / 300 tokens 106 / 150 -> 78.4 / 116 us, gate|up (9728 x
+// 896) at 700 tokens 35.1 -> 28.0 us.
+//
+// From 512 tiles of 128 x 128 those are taken outright (they win there), so the
+// choice and its partials repeat with every 512 token tiles.
+struct GemmCost {
+  int bm, bn, nst;
+  double alone, beside, merge;
+};
+constexpr GemmCost kGemmCosts[] = {
+    {128, 128, 3, 0.82, 0.47, 4.9}, {128, 64, 3, 0.55, 0.23, 1.3}, {64, 64, 4, 0.31, 0.22, 0.0}};
+
 GemmShape gemm_shape(int64_t M, int N, int K, bool can_split) {
-  auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  GemmShape s{64, 64, 4, 4, 0, 0, 1};
-  if (tiles(128, 128) >= 512) s = {128, 128, 3, 4, 0, 0, 1};
-  else if (K >= 2048 && tiles(128, 64) >= 200) s = {128, 64, 3, 4, 0, 0, 1};
-  s.tiles = s.whole = tiles(s.bm, s.bn);
-  const int64_t slots = int64_t{kGemmCUs} * (kLdsPerCU / gemm_lds(s.bm, s.bn, s.nst));
-  const int64_t last = s.tiles - (s.tiles - 1) / slots * slots;  // tiles of the last round
-  if (can_split && 2 * last <= slots && last <= gemm::kMaxSplitTiles) {
-    const int steps = K / gemm::BK;
-    const int64_t sp = std::min<int64_t>(std::min<int64_t>(slots / last, 4), steps / 8);
-    if (sp > 1) {
-      s.splits = static_cast<int>(sp);
-      s.whole = s.tiles - last;
-    }
+  const int steps = K / gemm::BK;
+  // `n` tiles at once on every CU, the last layer part filled.
+  auto layers = [](double n) { return std::max(1.0, 0.6 * std::ceil(n) + 0.4 * n); };
+  GemmShape best{};
+  double best_us = 0;
+  for (const GemmCost& c : kGemmCosts) {
+    GemmShape s{c.bm, c.bn, c.nst, 4, 0, 0, 1};
+    s.tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    const int per_cu = kLdsPerCU / gemm_lds(c.bm, c.bn, c.nst);
+    const int64_t slots = int64_t{kGemmCUs} * per_cu;
+    const int64_t full = (s.tiles - 1) / slots * slots, x = s.tiles - full;  // tiles of the last round
+    auto step_us = [&](double n) { return c.alone + c.beside * (n - 1); };
+    s.whole = s.tiles;
+    double tail_us = steps * step_us(layers(static_cast<double>(x) / kGemmCUs));
+    for (int sp = 2; can_split && sp <= 4 && steps / 8 >= sp; ++sp)
+      for (const int64_t round : {slots, int64_t{kGemmCUs}}) {
+        const int64_t whole = (x - 1) / round * round, last = x - whole;
+        if (last > gemm::kMaxSplitTiles || whole + last * sp > slots) continue;
+        const double n = static_cast<double>(last * sp) / kGemmCUs;
+        const int part = (steps + sp - 1) / sp;
+        const double run_us = whole ? steps * step_us(static_cast<double>(whole) / kGemmCUs) + part * c.beside * n
+                                    : part * step_us(layers(n));
+        if (run_us + 2.5 + c.merge * n >= tail_us) continue;
+        tail_us = run_us + 2.5 + c.merge * n;
+        s.whole = full + whole;
+        s.splits = sp;
+      }
+    const double us = static_cast<double>(full / slots) * steps * step_us(per_cu) + tail_us;
+    if (!best.bm || us < best_us) best = s, best_us = us;
+    if (c.bm == 128 && c.bn == 128 && s.tiles >= 512) break;
   }
-  return s;
+  return best;
 }
 
 int64_t gemm_part_bytes(const GemmShape& s) {

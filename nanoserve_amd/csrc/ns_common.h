@@ -193,6 +193,33 @@ __device__ __forceinline__ u32x2 ds_read_tr16_b64_at(uint32_t a) {
   asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(a), "n"(OFF));
   return r;
 }
+template <int OFF>
+__device__ __forceinline__ u32x2 ds_read_b64_at(uint32_t a) {
+  static_assert(OFF >= 0 && OFF < 65536, "16-bit offset");
+  u32x2 r;
+  asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(r) : "v"(a), "n"(OFF));
+  return r;
+}
+template <int OFF>
+__device__ __forceinline__ uint32_t ds_read_b32_at(uint32_t a) {
+  static_assert(OFF >= 0 && OFF < 65536, "16-bit offset");
+  uint32_t r;
+  asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(r) : "v"(a), "n"(OFF));
+  return r;
+}
+// f(constant 0), ..., f(constant N - 1).
+template <int V>
+struct Const {
+  static constexpr int value = V;
+  __device__ constexpr operator int() const { return V; }
+};
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(Const<I>{});
+    static_for<N, I + 1>(f);
+  }
+}
 // Until at most N of the wave's LDS operations are pending (they complete in
 // order; other users of the counter only make it wait longer).
 template <int N>

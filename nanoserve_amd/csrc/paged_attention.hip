@@ -873,20 +873,6 @@ struct PrefillCfg {
   static_assert(KG == 1 || WC * NF * 64 * 4 <= RING, "merge buffer fits the ring");
 };
 
-// f(constant 0), ..., f(constant N - 1).
-template <int V>
-struct Const {
-  static constexpr int value = V;
-  __device__ constexpr operator int() const { return V; }
-};
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(Const<I>{});
-    static_for<N, I + 1>(f);
-  }
-}
-
 // Wait until at most N of this wave's vector-memory operations are pending,
 // drain its LDS operations, then barrier.  Written as one asm statement so the
 // compiler adds no wait of its own for the LDS loads still in flight.

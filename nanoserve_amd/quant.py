@@ -17,6 +17,7 @@ each weight tile once per 64- or 128-token tile.
 
 from __future__ import annotations
 
+import functools
 import itertools
 
 import torch
@@ -35,10 +36,11 @@ FUSED_MAX_ROWS = 128
 # "auto" takes the dequantise + library GEMM steps instead of the tiled GEMM
 # for layers whose K is at least LONG_K above LONG_K_TILED_MAX_ROWS rows, but
 # only inside a graph capture.  The tiled GEMM's time grows with its K steps
-# per workgroup, and past 1024 tokens the long-K layers get too few splits to
-# keep that count down: graph-replayed on MI355X, down_proj (K 4864, N 896,
-# residual) takes 33.1 / 33.9 us tiled / dequantise + hipBLASLt at 1024
-# tokens, 54.0 / 36.4 at 1280, 48.1 / 43.4 at 2048 and 77.1 / 60.9 at 4096.
+# per workgroup, and past 1024 tokens the long-K layers have too many tiles to
+# split that far: graph-replayed on MI355X, down_proj (K 4864, N 896, residual)
+# takes 31.0 / 33.4 us tiled / dequantise + hipBLASLt at 1088 tokens, 41.2 /
+# 39.3 at 2048 and 65.4 / 52.0 at 4096; K 8192, N 2048 67.7 / 64.0 at 1088 and
+# 99.5 / 83.1 at 2048; K 14336, N 3584 163 / 142 and 286 / 212.
 # Called eagerly, the steps' four to five launches and tensor ops cost more
 # host time than the single launch saves on the device: the c5 engine (eager
 # prefill chunks of up to 2048 tokens) measured TTFT p50 17.0-18.5 ms with
@@ -114,23 +116,25 @@ def quantize_int4_groupwise(w: torch.Tensor, group_size: int = 128):
     return packed, scale.squeeze(2).contiguous(), zero.squeeze(2).to(torch.uint8).contiguous()
 
 
-# The tiled GEMM's split layout depends on M only through its tile shape
-# (chosen from ceil(M/128) and ceil(M/64)) and through how many tiles its
-# last dispatch round holds.  Every shape switch happens below 512 token
-# tiles of 128 rows, and past that the 128 x 128 tiles' last round repeats
-# every 512 token tiles (two workgroups per CU on 256 CUs), so multiples of
-# 64 rows up to twice that cover every token count.
+# The tiled GEMM's split layout depends on M only through its tile counts
+# (ceil(M/128) and ceil(M/64) token tiles).  From 512 tiles of 128 x 128 it
+# always takes those, and their last round repeats every 512 token tiles (two
+# workgroups per CU on 256 CUs), so multiples of 64 rows up to twice that cover
+# every token count.
 _SPLITK_SCAN_ROWS = 2 * 512 * 128
 
 
+@functools.lru_cache(maxsize=256)
 def splitk_workspace_bytes(N: int, K: int) -> int:
     """Workspace bytes that cover every token count of an N x K layer.
 
     The fused kernel (1..FUSED_MAX_ROWS rows) splits K while its tiles are few;
     the tiled GEMM (above) splits the tiles of a last dispatch round that
-    leaves at least half of the device idle, which can happen at any token
-    count, so the scan runs over every multiple of 64 rows up to the point
-    where the GEMM's layouts repeat.
+    leaves slots of the device idle, which can happen at any token count, so
+    the scan runs over every multiple of 64 rows up to the point where the
+    GEMM's layouts repeat.  It depends on the two sizes alone and is kept by
+    them: a model's layers share a handful of sizes (2.9 ms a scan of 3584 x
+    14336, 0.6 ms of 896 x 896).
     """
     lib = _lib.load()
     rows = list(range(1, FUSED_MAX_ROWS + 1))

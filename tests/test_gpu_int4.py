@@ -587,6 +587,47 @@ def test_tiled_gemm_splits_the_last_rounds_tiles(dtype, N, K, M, epi):
         assert (err <= tol).all(), f"{what}: max err {err.max():.3e}"
 
 
+# (N, K, M): every way the tiled GEMM deals its tiles: all of them split, a
+# layer of one tile per CU whole and the tiles past it split (64 x 64: also two
+# layers), a full round whole and the rest split; each of the three tile shapes,
+# with ragged last token and feature tiles.  (1008, 1024, 4665) runs 128 x 128
+# tiles unsplit below two per CU.
+TILE_DEALS = [(896, 2048, 129), (1536, 2048, 129), (1536, 2048, 647), (3072, 2048, 647), (2064, 2048, 462),
+              (3072, 3072, 462), (2064, 2048, 1091), (3072, 3072, 721), (2064, 1024, 1922), (2064, 2048, 4032),
+              (1008, 1024, 4665)]
+
+
+@pytest.mark.parametrize("N,K,M", TILE_DEALS, ids=[f"{n}x{k}-M{m}" for n, k, m in TILE_DEALS])
+def test_tiled_gemm_deals_tiles_and_splits(N, K, M):
+    """Within one rounding of the oracle, identical on a repeated call on the same
+    workspace, the arrival counters back at zero, and nothing written past the
+    bytes the size function asks for."""
+    from nanoserve_amd import _lib
+
+    need = _lib.load().ns_int4_linear_splitk_workspace_size(M, N, K)
+    assert (need == 0) == ((N, K, M) == (1008, 1024, 4665))
+    print(f"tile deal N={N} K={K} M={M}", flush=True)
+    packed, s, z = (t.to(DEV) for t in _weights(N, K, 128, N + M))
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    res = torch.randn(M, N, generator=g).to(torch.bfloat16)
+    ws = torch.zeros(need + 4096, dtype=torch.uint8, device=DEV)
+    ws[need:] = 7
+    kw = dict(residual=res.to(DEV), workspace=ws)
+    first = int4_linear(x.to(DEV), packed, s, z, None, 128, **kw)
+    again = int4_linear(x.to(DEV), packed, s, z, None, 128, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(first, again)
+    assert need == 0 or not ws[:SPLITK_COUNTER_BYTES].any(), "arrival counters must be left at zero"
+    assert bool((ws[need:] == 7).all())
+    w = dequantize_int4_ref(packed.cpu().numpy(), s.cpu().numpy(), z.cpu().numpy(), 128, NAME[torch.bfloat16])
+    y = int4_linear_ref(x.float().numpy(), w, None)
+    want = _round(y, torch.bfloat16) + res.double().numpy()
+    tol = 2 * RTOL[torch.bfloat16] * (np.abs(y) + np.abs(res.double().numpy())) + 1e-5
+    err = np.abs(first.double().cpu().numpy() - want)
+    assert (err <= tol).all(), f"max err {err.max():.3e}"
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("N,K,gs", [(16, 1152, 128), (80, 1280, 256), (112, 4224, 128), (4592, 1152, 384),
                                     (4624, 1536, 128)],
