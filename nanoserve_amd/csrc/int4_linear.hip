@@ -797,7 +797,7 @@ __device__ __forceinline__ typename DT::vec8 pair_order(typename DT::vec8 v) {
 // chunk) and a ring of R code slots (one tile's chunk, 1 KiB, each), then
 // the scales and zero-point words of up to kStreamCols groups per feature row.
 constexpr int kStreamCols = 32;
-template <int NT, int FT, int WAVES, int R>
+template <int NT, int FT, int WAVES, int R, bool NORM>
 struct StreamCfg {
   static constexpr int X_B = NT * 4096;
   static constexpr int WAVE_B = X_B + R * 1024;
@@ -806,8 +806,10 @@ struct StreamCfg {
   static constexpr int SC_B = ROWS * kStreamCols * 4;
   static constexpr int ZP_B = ROWS * 16 * 4;
   static constexpr int RED_B = WAVES * FT * NT * 1024;
-  static constexpr int STREAM_B = WAVES * WAVE_B + SC_B + ZP_B;
-  static constexpr int LDS = STREAM_B > RED_B ? STREAM_B : RED_B;
+  static constexpr int NW_B = NORM ? WAVES * 256 : 0;           // each wave's slice of the norm weight
+  static constexpr int SS_B = NORM ? WAVES * NT * 16 * 4 : 0;   // the rows' sums of squares
+  static constexpr int STREAM_B = WAVES * WAVE_B + SC_B + ZP_B + NW_B;
+  static constexpr int LDS = STREAM_B > RED_B + SS_B ? STREAM_B : RED_B + SS_B;
   static_assert(R >= FT && R < DM * FT && R <= 16, "the waits below count on it");
   static_assert(LDS <= 160 * 1024 - 64, "one workgroup fits a CU");
 };
@@ -817,9 +819,9 @@ __device__ __forceinline__ void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <class DT, int NT, int FT, int WAVES, int R>
+template <class DT, int NT, int FT, int WAVES, int R, bool NORM>
 __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void int4_stream_kernel(Int4LinearParams p) {
-  using C = StreamCfg<NT, FT, WAVES, R>;
+  using C = StreamCfg<NT, FT, WAVES, R, NORM>;
   constexpr int ESZ = sizeof(typename DT::T);
   constexpr int TILES = FT * NT;  // 16x16 tiles of the result
   constexpr int XD = 4 * NT;      // loads of a chunk's x
@@ -838,6 +840,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void int4_stream_kernel(Int4
   char* const ring = xbuf + C::X_B;
   char* const sc = smem + WAVES * C::WAVE_B;
   char* const zp = sc + C::SC_B;
+  char* const nwbuf = zp + C::ZP_B + wave * 256;
 
   // Loader roles.  x: load d brings rows 4d .. 4d+3, 16-byte unit u of row r
   // at LDS unit u ^ r, so that an operand read (16 rows, one unit) meets every
@@ -860,6 +863,9 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void int4_stream_kernel(Int4
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[f][t] = floatx4{0.f, 0.f, 0.f, 0.f};
   const uint32_t magic = f16_magic_pair();
+  float ss[NT];  // NORM: this wave's slice of the rows' sums of squares
+#pragma unroll
+  for (int t = 0; t < NT; ++t) ss[t] = 0.f;
 
   // Group of chunk c (a chunk lies inside one group).
   auto group_of = [&](int c) -> int {
@@ -903,6 +909,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void int4_stream_kernel(Int4
     };
 
     if (n > 0) {
+      if constexpr (NORM)
+        dma_lds4_off(static_cast<const char*>(p.norm_weight) + wave * (128 * ESZ), 4 * static_cast<uint32_t>(lane), nwbuf);
       load_x(0);
 #pragma unroll
       for (int u = 0; u < R; ++u)
@@ -941,16 +949,34 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void int4_stream_kernel(Int4
 #pragma unroll
         for (int t = 0; t < NT; ++t)
           b[j][t] = __builtin_bit_cast(V8, ds_read_b128(xbuf + t * 4096 + row * 256 + (((4 * grp + j) ^ row) << 4)));
+      V8 nw[NORM ? 4 : 1];
+      if constexpr (NORM) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) nw[j] = __builtin_bit_cast(V8, ds_read_b128(nwbuf + 64 * grp + 16 * j));
+      }
       lds_wait_all();
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (NORM) lds_ready(nw[j]);
 #pragma unroll
         for (int t = 0; t < NT; ++t) lds_ready(b[j][t]);
+      }
       if constexpr (X_AHEAD) load_x(i + 1);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) b[j][t] = pair_order<DT>(b[j][t]);
+        for (int t = 0; t < NT; ++t) {
+          if constexpr (NORM) {  // the arithmetic and order of int4_linear_kernel
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float v = static_cast<float>(b[j][t][e]);
+              ss[t] = __builtin_fmaf(v, v, ss[t]);
+              b[j][t][e] = to_model<DT>(v * static_cast<float>(nw[j][e]));
+            }
+          } else {
+            b[j][t] = pair_order<DT>(b[j][t]);
+          }
+        }
       const uint32_t zsh = 8 * ((zrow + group_of(ph + wave + i * WAVES)) & 3u);
 #pragma unroll
       for (int f = 0; f < FT; ++f) {
@@ -974,7 +1000,8 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void int4_stream_kernel(Int4
         const float scale = __builtin_bit_cast(float, scw);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const V8 a = dequant8_pairs<DT>(codes[j], zb, zb16, scale, magic);
+          const V8 a = NORM ? dequant8_mix<DT>(codes[j], zb, scale, magic)
+                            : dequant8_pairs<DT>(codes[j], zb, zb16, scale, magic);
 #pragma unroll
           for (int t = 0; t < NT; ++t) acc[f][t] = mfma16x16x32(DT{}, a, b[j][t], acc[f][t]);
         }
@@ -1012,6 +1039,15 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void int4_stream_kernel(Int4
   for (int f = 0; f < FT; ++f)
 #pragma unroll
     for (int t = 0; t < NT; ++t) red[(wave * TILES + f * NT + t) * 64 + lane] = acc[f][t];
+  float* const nss = reinterpret_cast<float*>(smem + C::RED_B);
+  if constexpr (NORM) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      ss[t] += __shfl_xor(ss[t], 16);  // the four lane groups holding this row
+      ss[t] += __shfl_xor(ss[t], 32);
+      if (grp == 0) nss[(wave * NT + t) * 16 + row] = ss[t];
+    }
+  }
   __syncthreads();
   constexpr int OWN = (TILES + WAVES - 1) / WAVES;
   floatx4 y4[OWN];
@@ -1022,6 +1058,12 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void int4_stream_kernel(Int4
     if (i < TILES) {
 #pragma unroll
       for (int w = 0; w < WAVES; ++w) y4[o] += red[(w * TILES + i) * 64 + lane];
+      if constexpr (NORM) {
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) sum += nss[(w * NT + i % NT) * 16 + row];
+        y4[o] *= rsqrtf(sum / static_cast<float>(p.K) + p.norm_eps);
+      }
     }
   }
 
@@ -1139,14 +1181,65 @@ StreamShape stream_shape(int64_t M, int N, int K, bool can_split) {
   return best;
 }
 
+constexpr int64_t kGemmMinRows = 128;  // the fused kernel takes M up to here
+
+// The stream kernel with the RMSNorm (one chunk per wave, 32-token tiles), for
+// the wide projections behind a norm (gate|up).  int4_linear_kernel brings x
+// and the codes in strided loads, normalises x again in every pair of feature
+// tiles and, past 64 tokens, holds 64 of them a wave; here up to 5 feature
+// tiles share one normalised x.  The order of every sum is
+// int4_linear_kernel's, so results are the same to the bit.  What bounds it is
+// a chain: launch, first loads, the norm, ft tiles' dequantisation and products
+// (0.75-1.2 us a tile), reduction.
+//
+// Feature tiles by rounds * (2.6 + 1.25 ft) us, fitted to MI355X timings
+// (graph-replayed, weights from HBM, one workgroup per CU by its LDS): 9728 x
+// 896 at 64 tokens 17.4 / 14.9 / 15.4 / 10.9 us with 2 / 3 / 4 / 5 tiles, at 32
+// tokens 12.7 / 8.3 / 9.1 / 10.3; 4864 x 1024 at 64 11.4 / 7.9 / 8.5 / 9.6.
+#define NS_INT4_NORM_SHAPES(X) X(2) X(3) X(4) X(5)
+StreamShape norm_stream_shape(int64_t M, int N) {
+  const int tiles = N / 16, mtiles = static_cast<int>((M + 31) / 32);
+  StreamShape best{};
+  float best_cost = 0.f;
+  for (int ft = 2; ft <= 5; ++ft) {
+    const int gx = (tiles + ft - 1) / ft;
+    const float cost = static_cast<float>((gx * mtiles + kCUs - 1) / kCUs) * (2.6f + 1.25f * ft);
+    if (best.ft == 0 || cost < best_cost) {
+      best = {2, ft, 8, mtiles, gx, 1};
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+// Whether it takes a call with a norm.  int4_linear_kernel -> this, us: 9728 x
+// 896 fp16 at 17 / 32 / 48 / 64 / 100 / 128 tokens 8.7 / 8.7 / 10.9 / 12.9 /
+// 29.0 / 31.7 -> 8.0 / 8.3 / 10.6 / 10.9 / 19.3 / 19.1 (16 tokens 7.0; 6.9 at
+// best here, and slower below), 4864 x 1024 at 32 / 64 / 128 8.2 / 10.9 / 21.3
+// -> 6.7 / 7.9 / 10.4, 28672 x 1024 21.5 / 38.1 / 93.9 -> 17.0 / 27.7 / 51-53.
+// Small layers have nothing to share: 1152 x 896 at 32 / 64 tokens 4.1 / 5.2
+// against 6.3 / 6.4; past 64 tokens they win too, 7.9 -> 6.5.  With less than
+// seven chunks waves idle (2048 x 512 at 64 / 128: 4.1 / 5.9 against 5.3 / 5.4).
+bool norm_stream_takes(int64_t M, int N, int K, int group_size) {
+  return K / 128 >= 7 && group_size % 128 == 0 && M > 16 && M <= kGemmMinRows && N / 16 >= (M > 64 ? 72 : 256);
+}
+
 template <class DT>
 hipError_t launch_int4_stream(const Int4LinearParams& p, const StreamShape& s, hipStream_t stream) {
   void* args[] = {const_cast<Int4LinearParams*>(&p)};
   const void* fn = nullptr;
 #define NS_PICK(NT_, FT_, W_, R_)                  \
   if (s.nt == NT_ && s.ft == FT_ && s.waves == W_) \
-    fn = reinterpret_cast<const void*>(&int4_stream_kernel<DT, NT_, FT_, W_, R_>);
-  NS_INT4_STREAM_SHAPES(NS_PICK)
+    fn = reinterpret_cast<const void*>(&int4_stream_kernel<DT, NT_, FT_, W_, R_, false>);
+  if (!p.norm_weight) {
+    NS_INT4_STREAM_SHAPES(NS_PICK)
+  }
+#undef NS_PICK
+#define NS_PICK(FT_) \
+  if (s.ft == FT_) fn = reinterpret_cast<const void*>(&int4_stream_kernel<DT, 2, FT_, 8, FT_, true>);
+  if (p.norm_weight) {
+    NS_INT4_NORM_SHAPES(NS_PICK)
+  }
 #undef NS_PICK
   if (!fn) return hipErrorInvalidValue;
   const dim3 grid(static_cast<unsigned>(s.gx), static_cast<unsigned>(s.mtiles), static_cast<unsigned>(s.splits));
@@ -1188,7 +1281,6 @@ bool aligned(const void* q, uintptr_t a) { return reinterpret_cast<uintptr_t>(q)
 // last in the grid, so when the whole tiles fill the device for some rounds
 // the splits share out the last round's tiles over its otherwise idle slots.
 // --------------------------------------------------------------------------
-constexpr int64_t kGemmMinRows = 128;  // the fused kernel takes M up to here
 namespace gemm {
 constexpr int BK = 64;
 constexpr int WAVES = 4, THREADS = WAVES * 64;
@@ -1767,7 +1859,10 @@ int int4_linear_entry(void* out, const void* x, int64_t x_stride_row, const void
   // A 64-wide K step of the GEMM lies inside one group.
   const bool use_gemm = M > kGemmMinRows && !norm_weight && K % gemm::BK == 0 && group_size % gemm::BK == 0 &&
                         (!bias || aligned(bias, 8)) && aligned(zeros, 4) && small;
-  const bool use_stream = M <= kGemmMinRows && !norm_weight && stream_takes(K, group_size) && aligned(zeros, 4) && small;
+  const bool use_norm_stream =
+      norm_weight && norm_stream_takes(M, N, K, group_size) && aligned(zeros, 4) && small;
+  const bool use_stream =
+      M <= kGemmMinRows && !norm_weight && stream_takes(K, group_size) && aligned(zeros, 4) && small;
   int splits = 1;
   if (splitk && (use_gemm || M <= kGemmMinRows)) {
     const bool have = workspace && aligned(workspace, 256) && workspace_bytes >= splitk_bytes(M, N, K);
@@ -1793,8 +1888,8 @@ int int4_linear_entry(void* out, const void* x, int64_t x_stride_row, const void
     p.gemm_gh = static_cast<uint32_t>(group_size / 32);
     p.gemm_ghinv = p.gemm_gh == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + p.gemm_gh - 1) / p.gemm_gh);
     e = dtype == NS_DTYPE_F16 ? launch_int4_gemm<F16>(p, gs, s) : launch_int4_gemm<BF16>(p, gs, s);
-  } else if (use_stream) {
-    const StreamShape ss = stream_shape(M, N, K, splits > 1);
+  } else if (use_stream || use_norm_stream) {
+    const StreamShape ss = use_norm_stream ? norm_stream_shape(M, N) : stream_shape(M, N, K, splits > 1);
     p.stream_cg = static_cast<uint32_t>(group_size / 128);
     p.stream_cginv =
         p.stream_cg == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + p.stream_cg - 1) / p.stream_cg);

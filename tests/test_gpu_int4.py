@@ -669,3 +669,42 @@ def test_long_k_weight_stream(dtype, N, K, gs, M):
     tol = 4 * RTOL[dtype] * np.abs(a * uv) + 4 * RTOL[dtype] * np.abs(a * uv).max() * 1e-2 + 1e-4
     err = np.abs(act.double().cpu().numpy() - _round(a * uv, dtype))
     assert (err <= tol).all(), f"silu: max err {err.max():.3e}"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N,K,gs,M", [(4096, 896, 128, 17), (4112, 896, 896, 33), (9728, 896, 128, 64),
+                                      (8208, 1024, 256, 47), (1152, 896, 128, 65), (1168, 1024, 1024, 128)])
+def test_normed_weight_stream_matches_small_launches_bit_for_bit(dtype, N, K, gs, M):
+    """Wide projections behind an RMSNorm at 17-128 rows against 8-row launches of the same rows.
+
+    Sums run in the same order in both kernels.  N = 4096 and 1152 are the
+    first widths taken (up to and past 64 rows); 16 features more leave the
+    last workgroup's tiles partly empty.
+    """
+    g = torch.Generator().manual_seed(71)
+    packed = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, generator=g).to(DEV)
+    s = (torch.rand(N, K // gs, generator=g) * 0.01).to(DEV)
+    z = torch.randint(0, 16, (N, K // gs), dtype=torch.uint8, generator=g).to(DEV)
+    x = torch.randn(M, K + 8, generator=g).to(dtype).to(DEV)[:, :K]
+    x[3] = 0
+    x[M - 1] *= 100
+    b = (torch.randn(N, generator=g) * 0.1).to(dtype).to(DEV)
+    res = torch.randn(M, N, generator=g).to(dtype).to(DEV)
+    w = (1 + 0.1 * torch.randn(K, generator=g)).to(dtype).to(DEV)
+    for kw in ({}, {"silu_mul": True}, {"residual": res}):
+        def call(a, e):
+            args = {k: v[a:e] if k == "residual" else v for k, v in kw.items()}
+            return int4_linear(x[a:e], packed, s, z, b, gs, norm_weight=w, **args)
+        many, few = call(0, M), torch.cat([call(a, min(a + 8, M)) for a in range(0, M, 8)])
+        torch.cuda.synchronize()
+        assert torch.equal(many, few), sorted(kw)
+        if not kw:  # and against the oracle's steps in 64 bits, for the first and last rows
+            rows = torch.tensor([0, 1, M - 2, M - 1])
+            xd, wd = x[rows].double().cpu(), w.double().cpu()
+            rstd = torch.rsqrt((xd ** 2).mean(1, keepdim=True) + 1e-6)
+            wq = torch.from_numpy(np.asarray(dequantize_int4_ref(packed.cpu().numpy(), s.cpu().numpy(),
+                                                                 z.cpu().numpy(), gs, NAME[dtype]))).double()
+            want = rstd * (xd * wd) @ wq.t() + b.double().cpu()
+            # x * w rounds once per operand; the sum once at the end.
+            tol = RTOL[dtype] * ((rstd * (xd * wd)).abs() @ wq.abs().t() + want.abs()) + 1e-4
+            assert ((many[rows].double().cpu() - want).abs() <= tol).all()
