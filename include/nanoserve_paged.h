@@ -275,6 +275,17 @@ size_t ns_paged_attention_workspace_size(int num_seqs, int num_heads, int num_kv
                                          int64_t num_tokens, int is_decode_only);
 
 /*
+ * ns_paged_prefill_columns -- how many (query row, head) columns a workgroup
+ * of ns_paged_attention's MFMA prefill kernel holds for a batch with these
+ * host lengths and query offsets: 128, or the wide kernel's 384 (head_dim 64)
+ * or 256 (head_dim 128).  Host arithmetic only; without host lengths a call
+ * takes 128.  No counterpart in the reference.
+ */
+int ns_paged_prefill_columns(const void* seq_lens_host, int seq_lens_host_is_int64,
+                             const void* query_start_loc_host, int query_start_loc_host_is_int64,
+                             int num_seqs, int num_heads, int num_kv_heads, int head_dim);
+
+/*
  * ns_paged_decode_plan_size, ns_paged_decode_plan -- the decode work plan of
  * one step's metadata, built on the device.  No counterpart in the
  * reference; it is the device-side form of the launch schedule that the

@@ -105,6 +105,10 @@ SIGNATURES = {
     "ns_paged_attention_workspace_size": (c_size_t, [
         c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int64, c_int,
     ]),
+    "ns_paged_prefill_columns": (c_int, [
+        c_void_p, c_int, c_void_p, c_int,        # seq_lens_host, is_int64, query_start_loc_host, is_int64
+        c_int, c_int, c_int, c_int,              # S, Hq, Hkv, D
+    ]),
     "ns_paged_decode_plan_size": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),  # S, Hkv, D, bs, max_seq_len
     "ns_paged_decode_plan": (c_int, [
         c_void_p, c_size_t,                      # plan, bytes

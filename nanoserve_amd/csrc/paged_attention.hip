@@ -1660,23 +1660,49 @@ int64_t host_index(const void* a, int is64, int64_t i) {
   return is64 ? static_cast<const int64_t*>(a)[i] : static_cast<const int32_t*>(a)[i];
 }
 
-// Whether the batch's multi-row sequences take the wide prefill kernel: its
-// column blocks must fill the CUs, with the last round's loss small enough.
-// Graph-replayed on MI355X, us, narrow / wide (wide column blocks): D = 64
-// (14 / 2 heads, fp16) one prompt of 8192 tokens 219 / 271 (280), six of about
-// 1850 119 / 123 (412), eight 151 / 143 (546), one of 16000 695 / 628 (546).
-// D = 128 (28 / 4 heads, bf16) one prompt of 2600 112 / 118 (268), 3000 141.5
-// / 134 (308), 4000 213 / 176.5 (412), two of about 3700 421 / 337 (852), one
-// of 16000 2302 / 1810 (1636).  A single round does too at D = 128 if its
-// blocks are about as long as each other (the longest sets the span): two
-// chunks of 1024 behind up to 8000 keys 349 / 312 (224), against one prompt of
-// 2048, whose blocks grow from nothing, 76 / 96 (212).  Chunks that leave much
-// of a wide block empty keep the narrow one.
+// Whether the batch's multi-row sequences take the wide prefill kernel.  It
+// shares a K/V tile among more columns, so a CU's time per column is shorter,
+// but makes fewer and longer workgroups: it loses where they leave CUs idle or
+// where one of them, the longest, sets the span.  Graph-replayed on MI355X, us
+// narrow / wide (wide column blocks), b2: two prompts or chunks, b4: four.
+//
+// D = 128 (28 / 4 heads, bf16; "g8": 16 / 2 heads).  Above 256 blocks the
+// narrow kernel's twice as many need a third round:
+//  - chunks behind a context win from there on: 2450 rows behind 300 / 1000 /
+//    3000 keys 124 / 119, 169 / 140, 301 / 261 (268), b2 1220 behind 300 86 / 74
+//    (272);
+//  - a whole prompt's last blocks hold few keys, so its third round costs
+//    little and the longest block counts: 2600 tokens 112 / 114 (288), g8 4600
+//    170 / 179 (288), g8 4800 181 / 185 (300); 2800 129 / 120 (308), g8 5000 192
+//    / 192 (314), 4000 205 / 164 (440).  The line lies at 308 blocks where one
+//    sequence makes most of them; b2 1400 80 / 72 (304) starts the second
+//    prompt's long blocks late, as b4 650 53 / 42 (280) does.
+// From 192 to 256 blocks a single round of wide ones runs as long as its
+// longest, two rounds of narrow ones as long as twice the mean, and longer with
+// more sequences, whose long blocks start late.  One sequence needs a mean of
+// 0.75 of the longest (2048 rows behind 1000 / 2000 / 4000 keys, 0.66 / 0.75 /
+// 0.83: 116 / 126, 163 / 161, 252 / 230; 224), two 0.70 (b2 1024 behind 500 /
+// 1000 / 2000, 0.63 / 0.69 / 0.75: 72 / 74, 90.5 / 90.4, 130 / 125; 224), more
+// 0.60 (b4 512 behind 300 / 1000, 0.61 / 0.70: 53 / 48, 77 / 73; 224).  Decode
+// rows beside them leave the lines where they are: one prompt of 2700 with 1 /
+// 16 / 48 of them 136 / 132, 141 / 135, 150 / 135 (296), b2 1024 behind 4000 227
+// / 211, 232 / 212, 243 / 217 (224), 2048 behind 4000 269 / 247, 275 / 248, 288 /
+// 251 (224), one prompt of 2048 88 / 107, 97 / 107, 105 / 109 (224).
+//
+// D = 64 (fp16, 14 / 2 heads; "g16": 32 / 2): from 512 blocks, two full rounds
+// (one prompt of 8192 217 / 265 (300), 14000 554 / 485 (512), 16000 720 / 671
+// (584); six, eight, ten of about 1850 97 / 104 (404), 130 / 129 (536), 156 / 151
+// (664)).  Blocks of about the same length pay for a third round in full, so
+// they need it two fifths filled: 14100 rows behind 10000 keys 1399 / 1421
+// (516), 18000 1841 / 1780 (658), g16 6800 behind 8000 994 / 1029 (568), 7500
+// 1148 / 1094 (626).
+//
+// Chunks that leave much of a wide block empty keep the narrow one.
 bool prefill_wide(const void* lens, int lens64, const void* qsl, int qsl64, int num_seqs, int group, int num_kv_heads,
                   int head_dim) {
   const int64_t cols = head_dim == 64 ? PrefillCfg<64, true>::COLS : PrefillCfg<128, true>::COLS;
-  int64_t blocks = 0, used = 0;   // column blocks, and the columns in them
-  double total = 0, longest = 0;  // keys
+  int64_t blocks = 0, used = 0, most = 0;  // column blocks, the columns in them, the most blocks of a sequence
+  double total = 0, longest = 0;           // keys
   for (int i = 0; i < num_seqs; ++i) {
     const int64_t ql = host_index(qsl, qsl64, i + 1) - host_index(qsl, qsl64, i);
     if (ql <= 1) continue;
@@ -1684,12 +1710,18 @@ bool prefill_wide(const void* lens, int lens64, const void* qsl, int qsl64, int 
     const double L = static_cast<double>(host_index(lens, lens64, i));
     blocks += n;
     used += ql * group * num_kv_heads;
+    most = n > most ? n : most;
     total += n * (L - 0.5 * ql);
     longest = L > longest ? L : longest;
   }
   if (used < 0.6 * cols * blocks) return false;
-  if (head_dim == 64) return blocks >= 512;
-  return blocks >= 288 || (blocks >= 192 && total >= 0.6 * longest * blocks);
+  // Whether a mean block holds at least `share` of the longest one's keys.
+  auto even = [&](double share) { return total >= share * longest * blocks; };
+  if (head_dim == 64) return blocks >= 620 || (blocks >= 512 && !even(0.68));
+  const bool one = most > 0.75 * blocks;
+  if (blocks >= 288) return blocks >= 308 || !one || even(0.52);
+  if (blocks > 256) return even(0.6);
+  return blocks >= 192 && even(one ? 0.75 : most > 0.4 * blocks ? 0.70 : 0.60);
 }
 
 // Fill pp.plan with the prefill schedule from host query offsets and lengths:
@@ -1774,6 +1806,23 @@ int build_prefill_plan(PrefillParams& pp, const void* lens, int lens64, const vo
   }
 }
 
+// Width and schedule of a batch's prefill rows from host lengths and query
+// offsets, into pp (group, num_kv_heads and max_ctx set) and grid_x;
+// `part_bytes` of split state are at hand.
+void plan_prefill(PrefillParams& pp, const void* lens, int lens64, const void* qsl, int qsl64, int num_seqs,
+                  int head_dim, size_t part_bytes, int& grid_x) {
+  pp.wide = prefill_wide(lens, lens64, qsl, qsl64, num_seqs, pp.group, pp.num_kv_heads, head_dim);
+  const bool d64 = head_dim == 64;
+  const int cols = pp.wide ? (d64 ? PrefillCfg<64, true>::COLS : PrefillCfg<128, true>::COLS)
+                           : PrefillCfg<64, false>::COLS;
+  const int mkeys = pp.wide || !d64 ? 64 : 128;  // KG * KT
+  const size_t slot = !pp.wide ? prefill_slot_bytes(head_dim)
+                               : (d64 ? PrefillCfg<64, true>::SLOT_BYTES : PrefillCfg<128, true>::SLOT_BYTES);
+  pp.plan_n = build_prefill_plan(pp, lens, lens64, qsl, qsl64, num_seqs, cols, mkeys,
+                                 static_cast<int>(part_bytes / slot), grid_x);
+  if (!pp.plan_n) pp.wide = 0;
+}
+
 }  // namespace
 }  // namespace ns
 
@@ -1806,6 +1855,25 @@ extern "C" size_t ns_paged_attention_workspace_size(int num_seqs, int num_heads,
   const ns::DecodeShape d =
       ns::decode_shape(num_seqs, num_kv_heads, ns::round_up_ctx(max_seq_len, block_size), head_dim, ns::kPlanCUs);
   return ns::workspace_layout(num_heads / num_kv_heads, head_dim, d.item_cap, !is_decode_only).total;
+}
+
+extern "C" int ns_paged_prefill_columns(const void* seq_lens_host, int seq_lens_host_is_int64,
+                                        const void* query_start_loc_host, int query_start_loc_host_is_int64,
+                                        int num_seqs, int num_heads, int num_kv_heads, int head_dim) {
+  using namespace ns;
+  if (!seq_lens_host || !query_start_loc_host || num_seqs <= 0 || num_kv_heads <= 0 || num_heads <= 0 ||
+      num_heads % num_kv_heads)
+    return NS_ERR_INVALID_ARG;
+  if ((head_dim != 64 && head_dim != 128) || num_heads / num_kv_heads > 16) return NS_ERR_UNSUPPORTED;
+  PrefillParams pp;
+  pp.group = num_heads / num_kv_heads;
+  pp.num_kv_heads = num_kv_heads;
+  pp.max_ctx = 0x7FFFFFFF;
+  int grid_x = 0;
+  plan_prefill(pp, seq_lens_host, seq_lens_host_is_int64, query_start_loc_host, query_start_loc_host_is_int64,
+               num_seqs, head_dim, kPrefillSlots * prefill_slot_bytes(head_dim), grid_x);
+  if (!pp.wide) return PrefillCfg<64, false>::COLS;
+  return head_dim == 64 ? PrefillCfg<64, true>::COLS : PrefillCfg<128, true>::COLS;
 }
 
 extern "C" size_t ns_paged_decode_plan_size(int num_seqs, int num_kv_heads, int head_dim, int block_size,
@@ -2056,20 +2124,9 @@ int paged_attention_entry(void* out, const void* query, const void* k_cache, con
     static_cast<AttnParams&>(pp) = p;
     pp.plan_n = 0;
     pp.wide = 0;
-    if (seq_lens_host && qsl_host) {
-      pp.wide = prefill_wide(seq_lens_host, seq_lens_host_is_int64, qsl_host, query_start_loc_host_is_int64, num_seqs,
-                             group, num_kv_heads, head_dim);
-      const bool d64 = head_dim == 64;
-      const int cols = pp.wide ? (d64 ? PrefillCfg<64, true>::COLS : PrefillCfg<128, true>::COLS)
-                               : PrefillCfg<64, false>::COLS;
-      const int mkeys = pp.wide || !d64 ? 64 : 128;  // KG * KT
-      const size_t slot = !pp.wide ? prefill_slot_bytes(head_dim)
-                                   : (d64 ? PrefillCfg<64, true>::SLOT_BYTES : PrefillCfg<128, true>::SLOT_BYTES);
-      pp.plan_n = build_prefill_plan(pp, seq_lens_host, seq_lens_host_is_int64, qsl_host,
-                                     query_start_loc_host_is_int64, num_seqs, cols, mkeys,
-                                     static_cast<int>(wl.pf_part_bytes / slot), pf_grid_x);
-      if (!pp.plan_n) pp.wide = 0;
-    }
+    if (seq_lens_host && qsl_host)
+      plan_prefill(pp, seq_lens_host, seq_lens_host_is_int64, qsl_host, query_start_loc_host_is_int64, num_seqs,
+                   head_dim, wl.pf_part_bytes, pf_grid_x);
   }
 
   hipStream_t st = static_cast<hipStream_t>(stream);
