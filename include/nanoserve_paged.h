@@ -54,6 +54,11 @@ extern "C" {
 #define NS_EPILOGUE_RESIDUAL 1
 #define NS_EPILOGUE_SILU_MUL 2
 
+/* Kernels of ns_int4_linear (ns_int4_linear_kernel). */
+#define NS_INT4_REGISTER 0 /* operands loaded into registers, one weight tile per 16 or 64 tokens */
+#define NS_INT4_STREAM 1   /* operands through LDS, up to 128 tokens */
+#define NS_INT4_TILED 2    /* tiled GEMM, more than 128 tokens */
+
 /* Human-readable text for a status code (static storage, never NULL). */
 const char* ns_error_string(int code);
 
@@ -187,6 +192,18 @@ int ns_int4_linear_splitk(void* out, const void* x, int64_t x_stride_row,
                           const void* residual, int epilogue, const void* norm_weight, float norm_eps,
                           int64_t M, int N, int K, int group_size, int dtype,
                           void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * ns_int4_linear_kernel -- which kernel ns_int4_linear (or, with
+ * has_workspace, ns_int4_linear_splitk given its workspace) runs for these
+ * sizes when its pointers meet the alignment of the faster kernels (zeros 4
+ * bytes, bias 8) and its operands 32-bit offsets: NS_INT4_REGISTER,
+ * NS_INT4_STREAM or NS_INT4_TILED, with the token rows and features of a
+ * workgroup's tile and the K splits (of the tiles that split).  Host
+ * arithmetic only.  No counterpart in the reference.
+ */
+int ns_int4_linear_kernel(int64_t M, int N, int K, int group_size, int has_norm, int has_workspace,
+                          int* tokens, int* features, int* splits);
 
 /*
  * ns_int4_linear_rope_cache -- the q|k|v projection of one attention layer

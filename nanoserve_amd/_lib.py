@@ -33,6 +33,10 @@ NS_EPILOGUE_NONE = 0
 NS_EPILOGUE_RESIDUAL = 1
 NS_EPILOGUE_SILU_MUL = 2
 
+NS_INT4_REGISTER = 0
+NS_INT4_STREAM = 1
+NS_INT4_TILED = 2
+
 DTYPE_CODES = {
     torch.float32: NS_DTYPE_F32,
     torch.float16: NS_DTYPE_F16,
@@ -79,6 +83,11 @@ SIGNATURES = {
         c_int64, c_int, c_int, c_int,            # M, N, K, group_size
         c_int,                                   # dtype
         c_void_p, c_size_t, c_void_p,            # workspace, bytes, stream
+    ]),
+    "ns_int4_linear_kernel": (c_int, [
+        c_int64, c_int, c_int, c_int,            # M, N, K, group_size
+        c_int, c_int,                            # has_norm, has_workspace
+        c_void_p, c_void_p, c_void_p,            # out: tile tokens, tile features, splits (int32 each)
     ]),
     "ns_int4_linear_rope_cache": (c_int, [
         c_void_p, c_void_p, c_int64,             # q_out, x, x row stride

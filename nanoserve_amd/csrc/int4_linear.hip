@@ -1197,7 +1197,7 @@ constexpr int64_t kGemmMinRows = 128;  // the fused kernel takes M up to here
 // 896 at 64 tokens 17.4 / 14.9 / 15.4 / 10.9 us with 2 / 3 / 4 / 5 tiles, at 32
 // tokens 12.7 / 8.3 / 9.1 / 10.3; 4864 x 1024 at 64 11.4 / 7.9 / 8.5 / 9.6.
 #define NS_INT4_NORM_SHAPES(X) X(2) X(3) X(4) X(5)
-StreamShape norm_stream_shape(int64_t M, int N) {
+StreamShape norm_stream_shape(int64_t M, int N, float* us = nullptr) {
   const int tiles = N / 16, mtiles = static_cast<int>((M + 31) / 32);
   StreamShape best{};
   float best_cost = 0.f;
@@ -1209,19 +1209,38 @@ StreamShape norm_stream_shape(int64_t M, int N) {
       best_cost = cost;
     }
   }
+  if (us) *us = best_cost + 1.f;  // measured 0 to 1.4 above the rounds
   return best;
 }
 
-// Whether it takes a call with a norm.  int4_linear_kernel -> this, us: 9728 x
-// 896 fp16 at 17 / 32 / 48 / 64 / 100 / 128 tokens 8.7 / 8.7 / 10.9 / 12.9 /
-// 29.0 / 31.7 -> 8.0 / 8.3 / 10.6 / 10.9 / 19.3 / 19.1 (16 tokens 7.0; 6.9 at
-// best here, and slower below), 4864 x 1024 at 32 / 64 / 128 8.2 / 10.9 / 21.3
-// -> 6.7 / 7.9 / 10.4, 28672 x 1024 21.5 / 38.1 / 93.9 -> 17.0 / 27.7 / 51-53.
-// Small layers have nothing to share: 1152 x 896 at 32 / 64 tokens 4.1 / 5.2
-// against 6.3 / 6.4; past 64 tokens they win too, 7.9 -> 6.5.  With less than
-// seven chunks waves idle (2048 x 512 at 64 / 128: 4.1 / 5.9 against 5.3 / 5.4).
+// Whether it takes a call with a norm, from 25 widths x 11 token counts with
+// either kernel forced (fp16, silu-mul epilogue; us int4_linear_kernel / this).
+// Past 64 tokens that one holds 64 of them a wave, and this wins at every width
+// (1152 x 896 at 65 / 128 tokens 7.6 / 6.5 and 7.7 / 6.5, 9728 x 896 at 128 30.5 /
+// 18.4; below 1152 not taken).  Up to 64 tokens int4_linear_kernel takes about
+// 2.1 us (seven chunks) or 2.45 (eight) for each round of its workgroups of 32
+// features x 16 tokens, and 1.6 or 3.3 besides; this one, whose workgroups
+// hold 32 tokens, computes a fourth for nothing at 33 to 48 and leaves part of its own
+// rounds empty.  K = 896: 4096 wide at 32 tokens 5.5 / 6.55 (not taken),
+// 9728 at 32 / 48 / 64 8.4 / 7.65, 10.4 / 9.9 and 12.4 / 9.9, 4864 at 48 6.7 / 7.6
+// (not), 14336 at 32 / 48 / 64 10.4 / 8.65, 14.1 / 14.9 (not) and 16.8 / 15.2,
+// 28672 at 48 23.8 / 27.2 (not); K = 1024: 4096 at 32 5.9 / 6.7 (not), 4864 at 32 /
+// 48 / 64 8.2 / 6.7, 8.4 / 7.7 and 10.8 / 7.7.  Widths below 4096 have nothing to share
+// (1152 x 896 at 32 4.0 / 6.0).  With less than seven chunks waves idle (2048 x
+// 512 at 64 / 128: 4.1 / 5.9 against 5.3 / 5.4).
+//
+// 16-token tiles, up to 16 tokens, would win at K = 1024 (4864 wide 6.2 -> 5.5,
+// 28672 13.9 -> 12.5 at 16 tokens) but not at 9728 x 896 (7.0 -> 6.9, and
+// slower below 16), and past 64 tokens in narrow layers (1152 x 896 at 100: 5.4
+// against the 6.4 taken); they are not built.
 bool norm_stream_takes(int64_t M, int N, int K, int group_size) {
-  return K / 128 >= 7 && group_size % 128 == 0 && M > 16 && M <= kGemmMinRows && N / 16 >= (M > 64 ? 72 : 256);
+  if (K / 128 < 7 || group_size % 128 != 0 || M <= 16 || M > kGemmMinRows) return false;
+  if (M > 64) return N / 16 >= 72;
+  if (N / 16 < 256) return false;
+  const int64_t rounds = ((M + 15) / 16 * ((N + 31) / 32) + kCUs - 1) / kCUs;
+  float us = 0.f;
+  norm_stream_shape(M, N, &us);
+  return us < (K / 128 == 7 ? 1.6f + 2.1f * rounds : 3.3f + 2.45f * rounds);
 }
 
 template <class DT>
@@ -1812,6 +1831,18 @@ size_t splitk_bytes(int64_t M, int N, int K) {
   return static_cast<size_t>(bytes);
 }
 
+// The kernel of a call: the tiled GEMM and the stream address x, the codes and
+// the scales by 32-bit offsets and take whole words of the zero points
+// (`words`); the GEMM also reads bias four at a time (`bias4`) and does not
+// fuse the RMSNorm, and a 64-wide K step of it lies inside one group.
+int int4_kernel(int64_t M, int N, int K, int group_size, bool norm, bool words, bool bias4) {
+  if (!words) return NS_INT4_REGISTER;
+  if (M > kGemmMinRows)
+    return !norm && K % gemm::BK == 0 && group_size % gemm::BK == 0 && bias4 ? NS_INT4_TILED : NS_INT4_REGISTER;
+  return (norm ? norm_stream_takes(M, N, K, group_size) : stream_takes(K, group_size)) ? NS_INT4_STREAM
+                                                                                       : NS_INT4_REGISTER;
+}
+
 int int4_linear_entry(void* out, const void* x, int64_t x_stride_row, const void* qweight, const void* scales,
                       const void* zeros, const void* bias, const void* residual, int epilogue,
                       const void* norm_weight, float norm_eps, int64_t M, int N, int K, int group_size, int dtype,
@@ -1850,21 +1881,13 @@ int int4_linear_entry(void* out, const void* x, int64_t x_stride_row, const void
   p.K = K;
   p.group_size = group_size;
   p.groups = K / group_size;
-  // The GEMM does not fuse the RMSNorm; its epilogue reads bias four at a time
-  // and its loads take whole 4-byte words of the zero-point table.
-  // Its loads address x, the codes and the scales by 32-bit byte offsets.
   const int64_t esz = 2, lim = int64_t{1} << 32;
-  const bool small = (M - 1) * x_stride_row * esz + int64_t{K} * esz < lim && int64_t{N} * (K / 2) < lim &&
-                     int64_t{N} * (K / group_size) * 4 < lim;
-  // A 64-wide K step of the GEMM lies inside one group.
-  const bool use_gemm = M > kGemmMinRows && !norm_weight && K % gemm::BK == 0 && group_size % gemm::BK == 0 &&
-                        (!bias || aligned(bias, 8)) && aligned(zeros, 4) && small;
-  const bool use_norm_stream =
-      norm_weight && norm_stream_takes(M, N, K, group_size) && aligned(zeros, 4) && small;
-  const bool use_stream =
-      M <= kGemmMinRows && !norm_weight && stream_takes(K, group_size) && aligned(zeros, 4) && small;
+  const bool words = aligned(zeros, 4) && (M - 1) * x_stride_row * esz + int64_t{K} * esz < lim &&
+                     int64_t{N} * (K / 2) < lim && int64_t{N} * (K / group_size) * 4 < lim;
+  const int kernel = int4_kernel(M, N, K, group_size, norm_weight, words, !bias || aligned(bias, 8));
+  const bool use_stream = kernel == NS_INT4_STREAM && !norm_weight;
   int splits = 1;
-  if (splitk && (use_gemm || M <= kGemmMinRows)) {
+  if (splitk && (kernel == NS_INT4_TILED || M <= kGemmMinRows)) {
     const bool have = workspace && aligned(workspace, 256) && workspace_bytes >= splitk_bytes(M, N, K);
     // A call whose plain kernel splits needs the workspace; the weight stream
     // runs unsplit without one.
@@ -1879,7 +1902,7 @@ int int4_linear_entry(void* out, const void* x, int64_t x_stride_row, const void
   }
   const hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e;
-  if (use_gemm) {
+  if (kernel == NS_INT4_TILED) {
     // The same shape splitk_layout sized the workspace for (or none split).
     const GemmShape gs = gemm_shape(M, N, K, splits > 1);
     p.gemm_gx = (N + gs.bn - 1) / gs.bn;
@@ -1888,8 +1911,8 @@ int int4_linear_entry(void* out, const void* x, int64_t x_stride_row, const void
     p.gemm_gh = static_cast<uint32_t>(group_size / 32);
     p.gemm_ghinv = p.gemm_gh == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + p.gemm_gh - 1) / p.gemm_gh);
     e = dtype == NS_DTYPE_F16 ? launch_int4_gemm<F16>(p, gs, s) : launch_int4_gemm<BF16>(p, gs, s);
-  } else if (use_stream || use_norm_stream) {
-    const StreamShape ss = use_norm_stream ? norm_stream_shape(M, N) : stream_shape(M, N, K, splits > 1);
+  } else if (kernel == NS_INT4_STREAM) {
+    const StreamShape ss = norm_weight ? norm_stream_shape(M, N) : stream_shape(M, N, K, splits > 1);
     p.stream_cg = static_cast<uint32_t>(group_size / 128);
     p.stream_cginv =
         p.stream_cg == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + p.stream_cg - 1) / p.stream_cg);
@@ -1908,6 +1931,31 @@ extern "C" int ns_int4_linear(void* out, const void* x, int64_t x_stride_row,
                               int64_t M, int N, int K, int group_size, int dtype, void* stream) {
   return ns::int4_linear_entry(out, x, x_stride_row, qweight, scales, zeros, bias, residual, epilogue, norm_weight,
                                norm_eps, M, N, K, group_size, dtype, stream, nullptr, 0, false);
+}
+
+extern "C" int ns_int4_linear_kernel(int64_t M, int N, int K, int group_size, int has_norm, int has_workspace,
+                                     int* tokens, int* features, int* splits) {
+  using namespace ns;
+  if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || !tokens || !features || !splits) return NS_ERR_INVALID_ARG;
+  if (N % 16 != 0 || K % 32 != 0 || group_size % 32 != 0 || K % group_size != 0 ||
+      (has_norm && (K % 128 != 0 || K / 128 > 8)))
+    return NS_ERR_UNSUPPORTED;
+  const int kernel = int4_kernel(M, N, K, group_size, has_norm, true, true);
+  *splits = 1;
+  if (kernel == NS_INT4_TILED) {
+    const GemmShape s = gemm_shape(M, N, K, has_workspace);
+    *tokens = s.bm, *features = s.bn, *splits = s.splits;
+  } else if (kernel == NS_INT4_STREAM) {
+    const StreamShape s = has_norm ? norm_stream_shape(M, N) : stream_shape(M, N, K, has_workspace);
+    *tokens = 16 * s.nt, *features = 16 * s.ft, *splits = s.splits;
+  } else {
+    const int mt = M <= 64 ? 16 : 64;
+    const int mtiles = static_cast<int>((M + mt - 1) / mt);
+    const Shape s = shape_for(static_cast<int>(M), N, K, mt, mtiles);
+    *tokens = mt, *features = 16 * s.ft;
+    if (has_workspace && M <= kGemmMinRows && s.batch > 1) *splits = splitk_for(N, K, mtiles);
+  }
+  return kernel;
 }
 
 extern "C" size_t ns_int4_linear_splitk_workspace_size(int64_t M, int N, int K) {

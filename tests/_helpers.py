@@ -4,12 +4,16 @@
 blocks (the reference's `build`, tests/test_paged_attention.py:39-65) and
 `make_md` builds metadata with int32 tables (test_paged_attention.py:68-94);
 both also take an index dtype so the engine's int64 contract is covered.
+`int4_kernel` asks the library which INT4 kernel a call takes.
 """
 
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
+from nanoserve_amd import _lib
 from nanoserve_amd.attention import AttentionMetadata
 
 
@@ -90,3 +94,12 @@ def md_to(md: AttentionMetadata, device) -> AttentionMetadata:
         seq_lens_cpu=md.seq_lens_cpu,
         query_start_loc_cpu=md.query_start_loc_cpu,
     )
+
+
+def int4_kernel(M, N, K, gs=128, norm=False, workspace=False):
+    """(kernel, tokens and features of a workgroup's tile, K splits) of an ns_int4_linear call."""
+    t, f, s = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
+    k = _lib.load().ns_int4_linear_kernel(M, N, K, gs, norm, workspace, ctypes.byref(t), ctypes.byref(f),
+                                          ctypes.byref(s))
+    assert k >= 0, k
+    return k, t.value, f.value, s.value

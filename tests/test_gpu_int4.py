@@ -15,12 +15,15 @@ import torch
 import torch.nn.functional as F
 
 from nanoserve_amd.quant import Int4Linear, int4_linear, quantize_int4_groupwise, quantize_model
+from nanoserve_amd import _lib
 from oracle.quant import dequantize_int4_ref, int4_linear_ref
+from tests._helpers import int4_kernel
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 RTOL = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}
 NAME = {torch.float16: "float16", torch.bfloat16: "bfloat16"}
+REGISTER, STREAM, TILED = _lib.NS_INT4_REGISTER, _lib.NS_INT4_STREAM, _lib.NS_INT4_TILED
 
 # Qwen2.5-0.5B projections (in -> out): q, k/v, o, gate/up, down, and fused q|k|v, gate|up.
 # Arrival-counter region at the head of every split-K workspace (256 tiles x u32).
@@ -673,14 +676,18 @@ def test_long_k_weight_stream(dtype, N, K, gs, M):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("N,K,gs,M", [(4096, 896, 128, 17), (4112, 896, 896, 33), (9728, 896, 128, 64),
-                                      (8208, 1024, 256, 47), (1152, 896, 128, 65), (1168, 1024, 1024, 128)])
+                                      (8208, 1024, 256, 47), (1152, 896, 128, 65), (1168, 1024, 1024, 128),
+                                      (4480, 1024, 128, 17), (4112, 1024, 512, 33), (6160, 896, 128, 62),
+                                      (7184, 896, 128, 50), (3088, 1024, 128, 97)])
 def test_normed_weight_stream_matches_small_launches_bit_for_bit(dtype, N, K, gs, M):
     """Wide projections behind an RMSNorm at 17-128 rows against 8-row launches of the same rows.
 
-    Sums run in the same order in both kernels.  N = 4096 and 1152 are the
-    first widths taken (up to and past 64 rows); 16 features more leave the
-    last workgroup's tiles partly empty.
+    Sums run in the same order in both kernels.  Every instantiated width of
+    2 to 5 feature tiles, with a last workgroup whose tiles are partly empty,
+    and the first widths taken (1152 past 64 rows, 4112 up to them); the two
+    rows that do not take the stream kernel are next to ones that do.
     """
+    assert int4_kernel(M, N, K, gs, norm=True)[0] == (REGISTER if K == 896 and M < 50 else STREAM)
     g = torch.Generator().manual_seed(71)
     packed = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, generator=g).to(DEV)
     s = (torch.rand(N, K // gs, generator=g) * 0.01).to(DEV)

@@ -1,0 +1,56 @@
+"""Which INT4 kernel a call takes: the one measured faster on each side of every line (no GPU needed).
+
+The times beside a case are of the register kernel and of the one named
+(MI355X, graph-replayed, weights from HBM, us), forced in turn.
+"""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+
+from nanoserve_amd import _lib
+from tests._helpers import int4_kernel
+
+REGISTER, STREAM, TILED = _lib.NS_INT4_REGISTER, _lib.NS_INT4_STREAM, _lib.NS_INT4_TILED
+
+
+@pytest.mark.parametrize("N,K,M,want", [
+    (4096, 896, 32, REGISTER),      # 5.50 / 6.55
+    (4096, 1024, 32, REGISTER),     # 5.90 / 6.71
+    (4096, 1024, 48, STREAM),       # 8.10 / 6.72
+    (4864, 896, 48, REGISTER),      # 6.72 / 7.62
+    (4864, 896, 64, STREAM),        # 8.25 / 7.66
+    (4864, 1024, 32, STREAM),       # 8.16 / 6.68
+    (6144, 896, 48, STREAM),        # 8.27 / 7.52
+    (9728, 896, 16, REGISTER),      # 6.98 / 6.90 at best, slower below
+    (9728, 896, 32, STREAM),        # 8.37 / 7.65
+    (9728, 896, 48, STREAM),        # 10.43 / 9.92
+    (9728, 896, 64, STREAM),        # 12.37 / 9.89
+    (9728, 896, 128, STREAM),       # 30.45 / 18.41
+    (11008, 896, 48, REGISTER),     # 11.99 / 13.60
+    (14336, 896, 48, REGISTER),     # 14.07 / 14.90
+    (14336, 896, 64, STREAM),       # 16.83 / 15.16
+    (24576, 896, 48, REGISTER),     # 20.93 / 23.15
+    (28672, 896, 48, REGISTER),     # 23.77 / 27.17
+    (28672, 896, 64, STREAM),       # 29.61 / 27.46
+    (28672, 1024, 48, STREAM),      # 30.36 / 27.48
+    (1152, 896, 32, REGISTER),      # 3.95 / 5.97
+    (1152, 896, 64, REGISTER),      # 4.98 / 6.47
+    (1152, 896, 65, STREAM),        # 7.62 / 6.48
+    (1152, 1024, 128, STREAM),      # 8.50 / 6.71
+    (1152, 896, 129, REGISTER),     # the tiled GEMM fuses no norm, the stream holds 128 rows
+])
+def test_projections_behind_a_norm_take_the_faster_kernel(N, K, M, want):
+    assert int4_kernel(M, N, K, norm=True)[0] == want
+
+
+def test_kernel_query_refuses_what_the_call_refuses():
+    lib = _lib.load()
+    t, f, s = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
+    out = (ctypes.byref(t), ctypes.byref(f), ctypes.byref(s))
+    assert lib.ns_int4_linear_kernel(0, 896, 896, 128, 0, 0, *out) == _lib.NS_ERR_INVALID_ARG
+    assert lib.ns_int4_linear_kernel(1, 896, 896, 128, 0, 0, None, *out[1:]) == _lib.NS_ERR_INVALID_ARG
+    for N, K, gs, norm in ((24, 896, 128, 0), (896, 900, 100, 0), (896, 896, 48, 0), (896, 1152, 128, 1)):
+        assert lib.ns_int4_linear_kernel(1, N, K, gs, norm, 0, *out) == _lib.NS_ERR_UNSUPPORTED
