@@ -1135,10 +1135,23 @@ struct StreamShape {
   int nt, ft, waves, mtiles, gx, splits;
 };
 
-// Whether the stream kernel takes the call: more chunks than the one-chunk
-// kernels hold, whole 128-wide chunks and each inside one group.
 constexpr int kCUs = 256;
-bool stream_takes(int K, int group_size) { return K > 1024 && K % 128 == 0 && group_size % 128 == 0; }
+
+// Whether the stream kernel takes the call: more chunks than the one-chunk
+// kernels hold, whole 128-wide chunks and each inside one group.  A few tokens
+// with 9, 11, 13 or 15 chunks stay with int4_linear_kernel while its one-tile
+// workgroups fit a few rounds: it is quicker at those counts than at the even
+// ones beside them, and its waves bring two chunks at once where the stream's
+// take one after the other.  us int4_linear_kernel / stream at 1 / 6 / 8 tokens:
+// 512 x 1152 3.5 / 3.8, 3.7 / 3.8 and 3.8 / 3.9; 12288 x 1152 5.6 / 6.6, 6.1 / 6.6
+// and 6.4 / 6.6; 8192 x 1664 5.9 / 6.3, 6.3 / 6.3 and 6.4 / 6.4; 16384 x 1152 8.5 /
+// 8.0, 10.1 / 7.9 and 10.7 / 7.9.  Even counts: 8192 x 1536 5.7 / 5.7, 6.2 / 5.7 and
+// 6.4 / 5.7; 12288 x 1280 6.3 / 6.7, 6.8 / 6.7 and 7.3 / 6.8; 512 x 1792 3.9 / 4.2,
+// 4.1 / 4.2 and 4.2 / 4.2.  From K = 2048 on the stream wins.
+bool stream_takes(int64_t M, int N, int K, int group_size) {
+  if (K <= 1024 || K % 128 != 0 || group_size % 128 != 0) return false;
+  return !(M <= 6 && K < 2048 && K % 256 != 0 && N < 16384);
+}
 
 // Instantiated shapes: (NT, FT, WAVES, R).
 #define NS_INT4_STREAM_SHAPES(X) \
@@ -1824,7 +1837,7 @@ static_assert(kSplitkCounterBytes % 256 == 0, "partials stay 256-byte aligned");
 size_t splitk_bytes(int64_t M, int N, int K) {
   const SplitkLayout l = splitk_layout(M, N, K, false);
   int64_t bytes = l.counter_bytes + l.part_bytes;
-  if (M <= kGemmMinRows && stream_takes(K, 128)) {
+  if (M <= kGemmMinRows && stream_takes(M, N, K, 128)) {
     const SplitkLayout ls = splitk_layout(M, N, K, true);
     bytes = std::max(bytes, ls.counter_bytes + ls.part_bytes);
   }
@@ -1839,7 +1852,7 @@ int int4_kernel(int64_t M, int N, int K, int group_size, bool norm, bool words, 
   if (!words) return NS_INT4_REGISTER;
   if (M > kGemmMinRows)
     return !norm && K % gemm::BK == 0 && group_size % gemm::BK == 0 && bias4 ? NS_INT4_TILED : NS_INT4_REGISTER;
-  return (norm ? norm_stream_takes(M, N, K, group_size) : stream_takes(K, group_size)) ? NS_INT4_STREAM
+  return (norm ? norm_stream_takes(M, N, K, group_size) : stream_takes(M, N, K, group_size)) ? NS_INT4_STREAM
                                                                                        : NS_INT4_REGISTER;
 }
 

@@ -46,6 +46,33 @@ def test_projections_behind_a_norm_take_the_faster_kernel(N, K, M, want):
     assert int4_kernel(M, N, K, norm=True)[0] == want
 
 
+@pytest.mark.parametrize("N,K,M,want", [
+    (512, 1152, 1, REGISTER),       # 3.48 / 3.81
+    (12288, 1152, 1, REGISTER),     # 5.57 / 6.58
+    (12288, 1152, 6, REGISTER),     # 6.08 / 6.58
+    (12288, 1152, 12, STREAM),      # 7.05 / 6.70
+    (16384, 1152, 1, STREAM),       # 8.54 / 7.98
+    (1536, 1408, 1, REGISTER),      # 4.05 / 4.21
+    (8192, 1664, 1, REGISTER),      # 5.92 / 6.34
+    (512, 1920, 1, REGISTER),       # 3.89 / 4.16
+    (512, 1536, 1, STREAM),         # 3.95 / 3.83
+    (8192, 1536, 6, STREAM),        # 6.17 / 5.69
+    (512, 2176, 1, STREAM),         # 5.99 / 4.31
+    (896, 4864, 1, STREAM),
+    (28672, 3584, 128, STREAM),
+    (896, 4864, 129, TILED),
+    (896, 896, 16, REGISTER),       # up to 1024 without a norm
+])
+def test_long_k_calls_take_the_faster_kernel(N, K, M, want):
+    assert int4_kernel(M, N, K)[0] == want
+
+
+@pytest.mark.parametrize("K,gs", [(4864, 64), (4864, 32), (4896, 32), (1280, 64)])
+def test_small_groups_and_part_chunks_keep_the_register_kernel(K, gs):
+    for M in (1, 16, 33, 128):
+        assert int4_kernel(M, 896, K, gs)[0] == REGISTER
+
+
 def test_kernel_query_refuses_what_the_call_refuses():
     lib = _lib.load()
     t, f, s = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
