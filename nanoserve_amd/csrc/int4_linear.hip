@@ -1684,26 +1684,31 @@ constexpr int gemm_lds(int bm, int bn, int nst) {
 // tiles split into 4-5 steps, 49.4 / 74.9 us against 39.5 / 64.9 unsplit), and
 // 2.5 us + `merge` per split a CU for the partials.  A part-filled layer of
 // tiles counts 0.6 as a full one: its chain is what the call waits for.
+// `start` is what an unsplit call's first loads and epilogue take longer than with
+// 64 x 64 tiles (the constants of a split hold it); without it calls of 14 to 24
+// steps took tiles that were too large (1152 x 896 at 2600 tokens 16.5 us with 128 x
+// 64 tiles, 15.6 with 64 x 64; 1024 x 1024 at 3000 17.9 / 17.0).
 //
-// The constants fit 54 layers and token counts with every shape and split
-// forced (MI355X, fp16, graph-replayed; 129 to 10000 tokens, 896 x 896 to
-// 28672 x 3584): the pick is the fastest in 43, within 5% in 52 and 11% behind
-// in two (1536 x 1536 and 2304 x 1536 at 1024 tokens, 18.6 / 22.5 us against
-// 16.7 / 20.2).  Against shapes by thresholds on the tile count and splits of a
-// last round only, both measured: down_proj (896 x 4864) at 512 / 1500 / 4700
-// tokens 24.4 / 50.4 / 112 -> 20.5 / 31.4 / 73.7 us, 3584 x 14336 at 200 / 800
-// / 1200 / 2000 tokens 74.7 / 176 / 313 / 366 -> 55.1 / 144 / 209 / 288 us,
-// 28672 x 3584 at 200 / 300 tokens 106 / 150 -> 78.4 / 116 us, gate|up (9728 x
-// 896) at 700 tokens 35.1 -> 28.0 us.
+// The constants fit 16 layers (512 x 512 to 2048 x 8192) at 25 token counts (200
+// to 4000) with each shape forced, with and without a workspace (MI355X, fp16,
+// graph-replayed): the pick is within 5% of the fastest in 792 of 800 and 14%
+// behind at worst (896 x 2048 at 1500 tokens, 22.6 / 19.7 us; 2048 x 2048 at 600,
+// 21.9 / 19.7).  Against shapes by thresholds on the tile count and splits of a
+// last round only, both measured: down_proj (896 x 4864) at 512 / 1500 / 4700 tokens 24.4 / 50.4 / 112 -> 20.5 / 31.4 / 73.7 us, 3584 x 14336 at
+// 200 / 800 / 1200 / 2000 tokens 74.7 / 176 / 313 / 366 -> 55.1 / 144 / 209 / 288
+// us, 28672 x 3584 at 200 / 300 tokens 106 / 150 -> 78.4 / 116 us, gate|up (9728 x
+// 896) at 700 tokens 35.1 -> 28.0 us; no call of the 800 is over 2.5% behind them.
 //
-// From 512 tiles of 128 x 128 those are taken outright (they win there), so the
-// choice and its partials repeat with every 512 token tiles.
+// From 512 tiles of 128 x 128 those are taken outright, so the choice and its
+// partials repeat with every 512 token tiles.  (They mostly win there, but not past
+// a full round by a little: 9728 x 896 at 800 tokens, 532 tiles, 43.5 us, against
+// 38.3 with 64 x 64.)
 struct GemmCost {
   int bm, bn, nst;
-  double alone, beside, merge;
+  double alone, beside, merge, start;
 };
 constexpr GemmCost kGemmCosts[] = {
-    {128, 128, 3, 0.82, 0.47, 4.9}, {128, 64, 3, 0.55, 0.23, 1.3}, {64, 64, 4, 0.31, 0.22, 0.0}};
+    {128, 128, 3, 0.82, 0.47, 4.9, 2.0}, {128, 64, 3, 0.55, 0.23, 1.3, 0.5}, {64, 64, 4, 0.31, 0.222, 0.0, 0.0}};
 
 GemmShape gemm_shape(int64_t M, int N, int K, bool can_split) {
   const int steps = K / gemm::BK;
@@ -1733,7 +1738,8 @@ GemmShape gemm_shape(int64_t M, int N, int K, bool can_split) {
         s.whole = full + whole;
         s.splits = sp;
       }
-    const double us = static_cast<double>(full / slots) * steps * step_us(per_cu) + tail_us;
+    const double us =
+        (s.splits > 1 ? 0 : c.start) + static_cast<double>(full / slots) * steps * step_us(per_cu) + tail_us;
     if (!best.bm || us < best_us) best = s, best_us = us;
     if (c.bm == 128 && c.bn == 128 && s.tiles >= 512) break;
   }

@@ -590,14 +590,17 @@ def test_tiled_gemm_splits_the_last_rounds_tiles(dtype, N, K, M, epi):
         assert (err <= tol).all(), f"{what}: max err {err.max():.3e}"
 
 
-# (N, K, M): every way the tiled GEMM deals its tiles: all of them split, a
-# layer of one tile per CU whole and the tiles past it split (64 x 64: also two
-# layers), a full round whole and the rest split; each of the three tile shapes,
-# with ragged last token and feature tiles.  (1008, 1024, 4665) runs 128 x 128
-# tiles unsplit below two per CU.
-TILE_DEALS = [(896, 2048, 129), (1536, 2048, 129), (1536, 2048, 647), (3072, 2048, 647), (2064, 2048, 462),
-              (3072, 3072, 462), (2064, 2048, 1091), (3072, 3072, 721), (2064, 1024, 1922), (2064, 2048, 4032),
-              (1008, 1024, 4665)]
+# (N, K, M) and the tile shape and splits taken: every way the tiled GEMM deals
+# its tiles: all of them split, a layer of one tile per CU whole and the tiles
+# past it split (64 x 64: also two layers), a full round whole and the rest
+# split, and none split; each of the three tile shapes, with ragged last token
+# and feature tiles.  (1008, 1024, 4828) runs 128 x 128 tiles unsplit below two
+# per CU.
+TILE_DEALS = {(896, 2048, 129): (64, 64, 4), (1536, 2048, 129): (64, 64, 3), (1536, 2048, 647): (64, 64, 2),
+              (3072, 2048, 647): (64, 64, 2), (2064, 2048, 462): (128, 64, 3), (3072, 3072, 462): (128, 64, 2),
+              (2064, 2048, 1091): (128, 64, 2), (3072, 3072, 721): (128, 128, 3), (2064, 1024, 1922): (128, 128, 2),
+              (2064, 2048, 4032): (128, 128, 4), (1008, 1024, 4665): (64, 64, 1), (1008, 1024, 4828): (128, 128, 1),
+              (2064, 1024, 1498): (128, 64, 1)}
 
 
 @pytest.mark.parametrize("N,K,M", TILE_DEALS, ids=[f"{n}x{k}-M{m}" for n, k, m in TILE_DEALS])
@@ -608,7 +611,8 @@ def test_tiled_gemm_deals_tiles_and_splits(N, K, M):
     from nanoserve_amd import _lib
 
     need = _lib.load().ns_int4_linear_splitk_workspace_size(M, N, K)
-    assert (need == 0) == ((N, K, M) == (1008, 1024, 4665))
+    assert int4_kernel(M, N, K, workspace=True) == (TILED, *TILE_DEALS[N, K, M])
+    assert (need == 0) == (TILE_DEALS[N, K, M][2] == 1)
     print(f"tile deal N={N} K={K} M={M}", flush=True)
     packed, s, z = (t.to(DEV) for t in _weights(N, K, 128, N + M))
     g = torch.Generator().manual_seed(M)

@@ -73,6 +73,24 @@ def test_small_groups_and_part_chunks_keep_the_register_kernel(K, gs):
         assert int4_kernel(M, 896, K, gs)[0] == REGISTER
 
 
+@pytest.mark.parametrize("N,K,M,tokens,features", [
+    (1152, 896, 2600, 64, 64),      # 15.6; 128 x 64 16.5
+    (1152, 896, 3600, 64, 64),      # 23.2; 128 x 64 26.6, 128 x 128 24.8
+    (1024, 1024, 2800, 64, 64),     # 16.7; 128 x 64 17.8
+    (1024, 1024, 3000, 64, 64),     # 17.0; 128 x 64 17.9
+    (2048, 1024, 1400, 64, 64),     # 17.0; 128 x 64 18.0
+    (2048, 1024, 2048, 128, 64),    # 18.7; 64 x 64 23.2
+    (1536, 1536, 1200, 64, 64),     # 18.5; 128 x 64 19.5
+    (1536, 1536, 2048, 64, 64),     # 23.0; 128 x 64 23.9
+    (3072, 896, 1400, 64, 64),      # 24.7; 128 x 128 25.6
+    (9728, 896, 2048, 128, 128),
+    (1536, 8960, 1800, 128, 64),
+])
+def test_the_tiled_gemm_takes_the_faster_tiles(N, K, M, tokens, features):
+    """Unsplit times per tile shape, us."""
+    assert int4_kernel(M, N, K)[:3] == (TILED, tokens, features)
+
+
 def test_kernel_query_refuses_what_the_call_refuses():
     lib = _lib.load()
     t, f, s = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
