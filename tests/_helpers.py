@@ -4,12 +4,13 @@
 blocks (the reference's `build`, tests/test_paged_attention.py:39-65) and
 `make_md` builds metadata with int32 tables (test_paged_attention.py:68-94);
 both also take an index dtype so the engine's int64 contract is covered.
-`int4_kernel` asks the library which INT4 kernel a call takes.
+`int4_kernel` and `prefill_columns` ask the library which kernel a call takes.
 """
 
 from __future__ import annotations
 
 import ctypes
+import itertools
 
 import torch
 
@@ -94,6 +95,15 @@ def md_to(md: AttentionMetadata, device) -> AttentionMetadata:
         seq_lens_cpu=md.seq_lens_cpu,
         query_start_loc_cpu=md.query_start_loc_cpu,
     )
+
+
+def prefill_columns(seqs, heads):
+    """Columns per prefill workgroup of a batch with these (context, new rows) sequences;
+    heads is (query heads, KV heads, head size)."""
+    lens = [c + q for c, q in seqs]
+    qsl = [0, *itertools.accumulate(q for _, q in seqs)]
+    return _lib.load().ns_paged_prefill_columns(
+        (ctypes.c_int64 * len(lens))(*lens), 1, (ctypes.c_int64 * len(qsl))(*qsl), 1, len(lens), *heads)
 
 
 def int4_kernel(M, N, K, gs=128, norm=False, workspace=False):

@@ -21,7 +21,7 @@ from nanoserve_amd.attention import _attention, _workspaces, prepare_decode_plan
 from nanoserve_amd.capture import graph_capture
 from nanoserve_amd.workloads import make_case, metadata_for
 from oracle.paged_attention import dense_reference, paged_attention_ref
-from tests._helpers import build_paged, make_md, md_to
+from tests._helpers import build_paged, make_md, md_to, prefill_columns
 
 pytestmark = pytest.mark.gpu
 
@@ -330,12 +330,14 @@ def test_prefill_wide_column_blocks(D, cols, dtype, block_size):
     """Batches with enough column blocks take the wide kernel (384 / 256 columns a
     workgroup): at least 512 blocks over 8 KV heads of 16 query heads, chunks of one
     row more and fewer than a block, of a few columns, of several blocks and of two
-    rows, contexts that end inside, at and just past a 64-key step, one past a
-    4096-entry table window (block size 1), and decode rows beside them."""
+    rows, contexts that end inside, at and just past a 64-key step, one of more than
+    4096 keys, which is split (and, at block size 1, past a table window in the narrow
+    call), and decode rows beside them."""
     rows = cols // 16
     qls = ([rows, rows - 1, rows + 1, 3 * rows] * 16)[:60] + [2, 5, 1, 1]
     seqs = [q + c for q, c in zip(qls, [0, 64 - rows, 65, 300, 1] * 13)]
     seqs[7] += 4096
+    assert prefill_columns([(n - m, m) for n, m in zip(seqs, qls)], (128, 8, D)) == cols
     q, kc, vc, md, _, _ = _case(seqs, qls, 128, 8, D, block_size, dtype)
     scale = 1.0 / math.sqrt(D)
     print(f"wide prefill D={D} bs={block_size}", flush=True)
@@ -343,6 +345,31 @@ def test_prefill_wide_column_blocks(D, cols, dtype, block_size):
     # Without host offsets the same call runs the narrow kernel over the full grid.
     md.seq_lens_cpu = md.query_start_loc_cpu = None
     _assert_close(_run(q, kc, vc, md, scale), paged_attention_ref(q, kc, vc, md, scale), dtype)
+
+
+@pytest.mark.parametrize("D,cols,dtype", [(64, 384, torch.float16), (128, 256, torch.bfloat16)])
+def test_prefill_wide_crosses_table_windows(D, cols, dtype):
+    """Block size 1 in the wide kernel: unsplit key ranges over two and three 4096-entry
+    table windows (64 steps each), with window edges inside a chunk's causal band, at its
+    first and last row and between two chunks' rows.  Equal blocks enough for the wide
+    kernel make an even share of the work longer than any of them, so none is split."""
+    rows = cols // 16 * (6 if D == 64 else 3)
+    seqs = [4096 + rows // 2, 4096, 4097, 4096 + rows, 4095 + rows, 4200, 8192 + rows // 2, 8193, 4160, 4500, 4096 + 64,
+            8300, 4400]
+    qls = [rows] * len(seqs)
+    batch = [(n - rows, rows) for n in seqs]
+    assert prefill_columns(batch, (128, 8, D)) == cols
+    blocks, steps = len(seqs) * 8 * rows * 16 // cols, [(n + 63) // 64 for n in seqs]
+    assert 2 * blocks // len(seqs) * (sum(steps) - len(steps) * (rows // 64 + 1)) // 256 > max(steps)
+    q, kc, vc, md, tables, _ = _case(seqs, qls, 128, 8, D, 1, dtype)
+    scale = 1.0 / math.sqrt(D)
+    print(f"wide prefill windows D={D}", flush=True)
+    got = _run(q, kc, vc, md, scale)
+    _assert_close(got, _run(q, kc, vc, make_md(seqs, qls, tables, 1, with_cpu_lists=False), scale), dtype, "narrow")
+    for i in (0, 7):  # two of the sequences against the oracle, by themselves
+        part = slice(i * rows, (i + 1) * rows)
+        one = make_md(seqs[i:i + 1], qls[:1], tables[i:i + 1], 1)
+        _assert_close(got[part], paged_attention_ref(q[part], kc, vc, one, scale), dtype, f"sequence {i}")
 
 
 @pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])

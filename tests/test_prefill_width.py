@@ -8,20 +8,13 @@ graph-replayed, us).
 from __future__ import annotations
 
 import ctypes
-import itertools
 
 import pytest
 
 from nanoserve_amd import _lib
+from tests._helpers import prefill_columns
 
 D64, G16, D128, G8 = (14, 2, 64), (32, 2, 64), (28, 4, 128), (16, 2, 128)  # query heads, KV heads, head size
-
-
-def _columns(seqs, heads):
-    lens = [c + q for c, q in seqs]
-    qsl = [0, *itertools.accumulate(q for _, q in seqs)]
-    return _lib.load().ns_paged_prefill_columns(
-        (ctypes.c_int64 * len(lens))(*lens), 1, (ctypes.c_int64 * len(qsl))(*qsl), 1, len(lens), *heads)
 
 
 def _chunks(n, rows, context):
@@ -76,12 +69,12 @@ def _chunks(n, rows, context):
 ])
 def test_the_faster_width_is_taken(seqs, heads, wide):
     want = {64: (128, 384), 128: (128, 256)}[heads[2]][wide]
-    assert _columns(seqs, heads) == want
+    assert prefill_columns(seqs, heads) == want
 
 
 def test_more_sequences_than_the_schedule_lists_take_the_narrow_kernel():
-    assert _columns([(0, 64)] * 256, (128, 8, 128)) == 256
-    assert _columns([(0, 64)] * 257, (128, 8, 128)) == 128
+    assert prefill_columns([(0, 64)] * 256, (128, 8, 128)) == 256
+    assert prefill_columns([(0, 64)] * 257, (128, 8, 128)) == 128
 
 
 def test_bad_arguments_are_refused():
