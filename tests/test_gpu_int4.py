@@ -465,17 +465,19 @@ def test_rope_cache_epilogue_matches_projection_then_rotary(dtype, M, heads, wit
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M", [1, 16, 33, 64, 100, 200, 700, 2048])
 def test_splitk_down_projection(dtype, M):
-    """ns_int4_linear_splitk on down_proj's shape (N 896, K 4864; 4 splits per
-    16-token tile up to 16 tokens, 2 up to 32, none at 33-64; beyond 64 tokens the
-    tiles are 64 tokens wide and split twice again; above 128 tokens the tiled GEMM
-    splits its 64 x 64 tiles 4 times up to 896 tokens and 3 times up to 1152, and
-    from 1793 tokens its 128 x 64 tiles twice): within one rounding of the oracle on
+    """ns_int4_linear_splitk on down_proj's shape (N 896, K 4864; up to 128 tokens the
+    weight stream with 3 splits up to 16 tokens and at 33, none at 64 and 2 at 100;
+    above, the tiled GEMM splits its 64 x 64 tiles 4 times at 200 and 700 tokens and its
+    128 x 64 tiles twice at 2048): within one rounding of the oracle on
     the residual epilogue, identical on a repeated call (the arrival counters are back
     at zero), identical rows for a batch and its first row alone when both split the
     same way, and within one rounding of the unsplit kernel."""
     from nanoserve_amd.quant import splitk_workspace_bytes
 
     N, K = 896, 4864
+    assert int4_kernel(M, N, K, workspace=True) == {
+        1: (STREAM, 16, 16, 3), 16: (STREAM, 16, 16, 3), 33: (STREAM, 16, 32, 3), 64: (STREAM, 16, 16, 1),
+        100: (STREAM, 32, 32, 2), 200: (TILED, 64, 64, 4), 700: (TILED, 64, 64, 4), 2048: (TILED, 128, 64, 2)}[M]
     packed, s, z = (t.to(DEV) for t in _weights(N, K, 128, 71))
     g = torch.Generator().manual_seed(72)
     x = torch.randn(M, K, generator=g).to(dtype)
@@ -509,9 +511,9 @@ def test_splitk_workspace_reused_across_token_counts(dtype):
     equals, bit for bit, the same call on a fresh zeroed workspace, and the whole
     arrival-counter region is back at zero after every call.  A small-M call's
     partial sums must never land where a larger-M call keeps its counters (the
-    300-token call splits every tile of the tiled GEMM, the 4700-token call the
-    tiles of its last dispatch round, the 1500-token call none; the rest split
-    in the fused kernel)."""
+    300- and 1500-token calls split every tile of the tiled GEMM, the 4700-token call
+    the tiles past one per CU, the 4097-token call none; the rest split in the weight
+    stream)."""
     from nanoserve_amd.quant import splitk_workspace_bytes
 
     N, K = 896, 4864
@@ -520,7 +522,9 @@ def test_splitk_workspace_reused_across_token_counts(dtype):
     shared = torch.zeros(nbytes, dtype=torch.uint8, device=DEV)
     g = torch.Generator().manual_seed(82)
     b = (torch.randn(N, generator=g) * 0.1).to(dtype).to(DEV)
-    for M in (1, 32, 300, 100, 1, 1500, 4700, 17, 8, 32):
+    splits = {1: 3, 32: 2, 300: 3, 100: 2, 1500: 3, 4097: 1, 4700: 2, 17: 2, 8: 3}
+    for M in (1, 32, 300, 100, 1, 1500, 4097, 4700, 17, 8, 32):
+        assert int4_kernel(M, N, K, workspace=True)[3] == splits[M]
         print(f"splitk reuse M={M} {dtype}", flush=True)
         x = torch.randn(M, K, generator=g).to(dtype).to(DEV)
         res = torch.randn(M, N, generator=g).to(dtype).to(DEV)
@@ -533,14 +537,13 @@ def test_splitk_workspace_reused_across_token_counts(dtype):
         assert not fresh_ws[:SPLITK_COUNTER_BYTES].any()
 
 
-# (N, K, M, epilogue): tiled-GEMM calls on long-K layers whose tiles take more
-# than one dispatch round with a part-filled last one, which the library splits
-# over K while the earlier rounds' tiles run whole.  down_proj at 4700 tokens:
-# 518 128 x 64 tiles on 512 slots, the last 6 (the partial token tile among
-# them) split 4 ways; at 10000 tokens: 553 128 x 128 tiles, the last 41 split 4
-# ways (residual epilogue); a 1152 x 2048 layer at 3700 tokens: 522 128 x 64
-# tiles, the last 10 split 4 ways (bias); a 9728 x 2048 gate|up at 800
-# tokens: 532 128 x 128 tiles, the last 20 split 4 ways (SiLU-mul).
+# (N, K, M, epilogue): tiled-GEMM calls on long-K layers whose 128 x 128 tiles
+# take more than one per CU with few past the last whole layer or round of
+# them, which the library splits over K while the others run whole.  down_proj at
+# 4700 tokens: 259 tiles, the last 3 (the partial token tile among them) split
+# twice; at 10000 tokens: 553 tiles, the last 41 split 4 ways (residual epilogue); a
+# 1152 x 2048 layer at 3700 tokens: 261 tiles, the last 5 split twice (bias); a 9728 x
+# 2048 gate|up at 800 tokens: 532 tiles, the last 20 split 4 ways (SiLU-mul).
 TAIL_SPLITS = [(896, 4864, 4700, "residual"), (896, 4864, 10000, "residual"), (1152, 2048, 3700, "bias"),
                (9728, 2048, 800, "silu")]
 
@@ -556,6 +559,7 @@ def test_tiled_gemm_splits_the_last_rounds_tiles(dtype, N, K, M, epi):
 
     lib = _lib.load()
     assert lib.ns_int4_linear_splitk_workspace_size(M, N, K) > SPLITK_COUNTER_BYTES, "the call must split"
+    assert int4_kernel(M, N, K, workspace=True) == (TILED, 128, 128, 4 if M in (10000, 800) else 2)
     print(f"tail split N={N} K={K} M={M} {epi} {dtype}", flush=True)
     packed, s, z = (t.to(DEV) for t in _weights(N, K, 128, N + M))
     g = torch.Generator().manual_seed(M)
@@ -644,11 +648,13 @@ def test_long_k_weight_stream(dtype, N, K, gs, M):
     """Decode-size calls on K > 1024 layers against the oracle: one and many feature
     tiles (a last workgroup with fewer tiles than the others), 9 to 33 chunks (one
     more than a scale table holds, and fewer than the waves after a split), groups of
-    one, two and three chunks, part-filled token tiles, strided x rows; and the split
+    one, two and three chunks, part-filled token tiles, strided x rows (one row of K =
+    1152 stays with the register kernel); and the split
     call (which rounds its partial sums in another order) within the same bound,
     with its counters back at zero."""
     from nanoserve_amd.quant import splitk_workspace_bytes
 
+    assert int4_kernel(M, N, K, gs)[0] == (REGISTER if K == 1152 and M == 1 else STREAM)
     print(f"stream M={M} N={N} K={K} gs={gs} {dtype}", flush=True)
     packed, s, z = (t.to(DEV) for t in _weights(N, K, gs, N + K))
     g = torch.Generator().manual_seed(M)
