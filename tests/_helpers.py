@@ -113,3 +113,27 @@ def int4_kernel(M, N, K, gs=128, norm=False, workspace=False):
                                           ctypes.byref(s))
     assert k >= 0, k
     return k, t.value, f.value, s.value
+
+
+# Every (tokens, features) of a workgroup of the weight stream without a norm,
+# whose waits and ring are compile-time functions of the two, with (N, K, M) that
+# take it: few chunks a wave, more chunks than a scale table holds (32 and one or
+# more), and split over K (a workspace given).  The last workgroup holds fewer
+# tiles than the others and the last token tile is part empty.
+INT4_STREAM_CASES = {
+    (16, 16): ((16, 1280, 1), (16, 4224, 1), (16, 3584, 1)),
+    (16, 32): ((528, 1280, 127), (528, 4224, 127), (272, 4224, 127)),
+    (16, 48): ((1040, 1280, 127), (1040, 4224, 127), (544, 3584, 127)),
+    (16, 64): ((2064, 1280, 100), (2064, 4224, 100), (688, 4224, 100)),
+    (16, 80): ((6208, 1280, 33), (6208, 4224, 33), (3088, 3584, 33)),
+    (16, 96): ((20528, 1280, 1), (20528, 4224, 1), (10928, 14336, 1)),
+    (16, 112): ((24608, 1280, 1), (24608, 4224, 1), (12368, 4352, 1)),
+    (16, 128): ((28688, 1280, 1), (28688, 4224, 1), (10288, 8192, 1)),
+    (32, 16): ((528, 8192, 127), (528, 8192, 127), (336, 6144, 127)),
+    (32, 32): ((1552, 1280, 127), (1552, 4224, 127), (528, 4224, 127)),
+    (32, 48): ((2080, 1280, 127), (2080, 4224, 127), (1040, 3584, 127)),
+    (32, 64): ((3088, 1280, 100), (3088, 4224, 100), (1040, 4224, 127)),
+    (32, 80): ((4128, 1280, 100), (4128, 4224, 100), (1552, 3584, 127)),
+    (32, 96): ((5168, 1280, 100), (5168, 4224, 100), (2576, 4864, 100)),
+    (32, 112): ((6208, 1280, 100), (6208, 4224, 100), (2064, 4224, 100)),
+}

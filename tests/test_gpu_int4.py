@@ -17,7 +17,7 @@ import torch.nn.functional as F
 from nanoserve_amd.quant import Int4Linear, int4_linear, quantize_int4_groupwise, quantize_model
 from nanoserve_amd import _lib
 from oracle.quant import dequantize_int4_ref, int4_linear_ref
-from tests._helpers import int4_kernel
+from tests._helpers import INT4_STREAM_CASES, int4_kernel
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -682,6 +682,58 @@ def test_long_k_weight_stream(dtype, N, K, gs, M):
     tol = 4 * RTOL[dtype] * np.abs(a * uv) + 4 * RTOL[dtype] * np.abs(a * uv).max() * 1e-2 + 1e-4
     err = np.abs(act.double().cpu().numpy() - _round(a * uv, dtype))
     assert (err <= tol).all(), f"silu: max err {err.max():.3e}"
+
+
+def _random_layer(N, K, gs, seed):
+    """Random codes, scales and zero points on the GPU, without quantising a weight."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    packed = torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, device=DEV, generator=g)
+    s = torch.rand(N, K // gs, device=DEV, generator=g) * 0.01
+    z = torch.randint(0, 16, (N, K // gs), dtype=torch.uint8, device=DEV, generator=g)
+    return packed, s, z, g
+
+
+def _guarded(M, N, dtype):
+    """An [M, N] output with 4096 elements of a known value behind it."""
+    buf = torch.full((M * N + 4096,), 7.0, dtype=dtype, device=DEV)
+    return buf[:M * N].view(M, N), buf[M * N:]
+
+
+def _check_features(got, x, packed, s, z, b, gs, dtype, what):
+    """One feature of every 16-feature tile, another position in each, and the whole last tile."""
+    N = packed.shape[0]
+    f = torch.cat([torch.arange(N // 16) * 16 + torch.arange(N // 16) * 7 % 16, torch.arange(N - 16, N)])
+    w = dequantize_int4_ref(packed.cpu()[f].numpy(), s.cpu()[f].numpy(), z.cpu()[f].numpy(), gs, NAME[dtype])
+    ref = int4_linear_ref(x.float().cpu().numpy(), w, b.float().cpu()[f].numpy())
+    _check(got.cpu()[:, f], ref, dtype, what)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tile", INT4_STREAM_CASES, ids=lambda t: f"{t[0]}x{t[1]}")
+def test_every_weight_stream_shape(tile, dtype):
+    """Each instantiated shape on few chunks a wave, on two table phases and split,
+    against the oracle, with the same bits on a repeated call, its arrival counters
+    back at zero and nothing written past the output or the workspace."""
+    for N, K, M in INT4_STREAM_CASES[tile]:
+        need = _lib.load().ns_int4_linear_splitk_workspace_size(M, N, K)
+        split = (N, K, M) == INT4_STREAM_CASES[tile][2]
+        assert int4_kernel(M, N, K, workspace=split)[:3] == (STREAM, *tile)
+        print(f"stream tile={tile} M={M} N={N} K={K} split={split} {dtype}", flush=True)
+        packed, s, z, g = _random_layer(N, K, 128, N + K)
+        x = torch.randn(M, K, device=DEV, generator=g).to(dtype)
+        b = (torch.randn(N, device=DEV, generator=g) * 0.1).to(dtype)
+        out, guard = _guarded(M, N, dtype)
+        ws = torch.zeros(need + 4096, dtype=torch.uint8, device=DEV) if split else None
+        if split:
+            ws[need:] = 7
+        first = int4_linear(x, packed, s, z, b, 128, out=out, workspace=ws).clone()
+        again = int4_linear(x, packed, s, z, b, 128, out=out, workspace=ws)
+        torch.cuda.synchronize()
+        assert torch.equal(first, again)
+        assert bool((guard == 7).all())
+        if split:
+            assert not ws[:SPLITK_COUNTER_BYTES].any() and bool((ws[need:] == 7).all())
+        _check_features(first, x, packed, s, z, b, 128, dtype, f"{tile} M={M} N={N} K={K}")
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

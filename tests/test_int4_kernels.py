@@ -11,7 +11,7 @@ import ctypes
 import pytest
 
 from nanoserve_amd import _lib
-from tests._helpers import int4_kernel
+from tests._helpers import INT4_STREAM_CASES, int4_kernel
 
 REGISTER, STREAM, TILED = _lib.NS_INT4_REGISTER, _lib.NS_INT4_STREAM, _lib.NS_INT4_TILED
 
@@ -89,6 +89,33 @@ def test_small_groups_and_part_chunks_keep_the_register_kernel(K, gs):
 def test_the_tiled_gemm_takes_the_faster_tiles(N, K, M, tokens, features):
     """Unsplit times per tile shape, us."""
     assert int4_kernel(M, N, K)[:3] == (TILED, tokens, features)
+
+
+def test_the_stream_cases_take_every_shape_the_rule_can_pick():
+    """The GPU tests run each of INT4_STREAM_CASES: they must take the shapes they
+    stand for, and no layer may take a shape that is not among them."""
+    for tile, (few, phases, split) in INT4_STREAM_CASES.items():
+        for N, K, M in (few, phases):
+            assert int4_kernel(M, N, K) == (STREAM, *tile, 1)
+        N, K, M = split
+        got = int4_kernel(M, N, K, workspace=True)
+        assert got[:3] == (STREAM, *tile) and got[3] > 1
+        assert phases[1] // 128 > 32
+    taken = set()
+    for K in (1152, 1280, 2048, 3584, 4864, 8192, 14336):
+        for N in [*range(16, 2048, 48), *range(2048, 30000, 208), 65536, 151936]:
+            for M in (1, 8, 16, 17, 32, 33, 48, 64, 65, 100, 128):
+                for workspace in (False, True):
+                    kind, *tile, _ = int4_kernel(M, N, K, workspace=workspace)
+                    if kind == STREAM:
+                        taken.add(tuple(tile))
+    assert taken == set(INT4_STREAM_CASES)
+
+
+def test_the_normed_stream_takes_two_to_five_feature_tiles():
+    taken = {int4_kernel(M, N, K, norm=True)[1:3] for K in (896, 1024) for N in range(1152, 30000, 112)
+             for M in (17, 32, 33, 48, 64, 65, 100, 128) if int4_kernel(M, N, K, norm=True)[0] == STREAM}
+    assert taken == {(32, 32), (32, 48), (32, 64), (32, 80)}
 
 
 def test_kernel_query_refuses_what_the_call_refuses():
