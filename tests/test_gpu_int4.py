@@ -737,6 +737,36 @@ def test_every_weight_stream_shape(tile, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("K,gs,M,splits", [(4864, 32, 1, 4), (4864, 64, 16, 4), (4896, 32, 1, 4), (4896, 32, 33, 1),
+                                           (4896, 32, 17, 2), (4864, 64, 100, 2), (4896, 32, 100, 2), (4864, 64, 33, 1),
+                                           (1280, 64, 16, 1), (1312, 32, 5, 1), (1152, 32, 100, 1)])
+def test_long_k_with_small_groups_or_part_chunks(K, gs, M, splits, dtype):
+    """Long K that the weight stream does not take (groups under 128, or 32-wide steps
+    past the last whole chunk): the register kernel's several chunks a wave, with 8 and 16
+    waves and 16- and 64-token tiles, whole and split over K: against the oracle, with the
+    same bits on a repeated call, its arrival counters back at zero and nothing written past
+    the output or the workspace."""
+    N = 896
+    need = _lib.load().ns_int4_linear_splitk_workspace_size(M, N, K)
+    assert int4_kernel(M, N, K, gs, workspace=True) == (REGISTER, 16 if M <= 64 else 64, 16, splits)
+    print(f"register M={M} N={N} K={K} gs={gs} {dtype}", flush=True)
+    packed, s, z, g = _random_layer(N, K, gs, K + gs)
+    x = torch.randn(M, K, device=DEV, generator=g).to(dtype)
+    b = (torch.randn(N, device=DEV, generator=g) * 0.1).to(dtype)
+    ws = torch.zeros(need + 4096, dtype=torch.uint8, device=DEV)
+    ws[need:] = 7
+    for w in (None, ws):
+        out, guard = _guarded(M, N, dtype)
+        first = int4_linear(x, packed, s, z, b, gs, out=out, workspace=w).clone()
+        again = int4_linear(x, packed, s, z, b, gs, out=out, workspace=w)
+        torch.cuda.synchronize()
+        assert torch.equal(first, again)
+        assert bool((guard == 7).all()) and bool((ws[need:] == 7).all())
+        assert need == 0 or not ws[:SPLITK_COUNTER_BYTES].any(), "arrival counters must be left at zero"
+        _check_features(first, x, packed, s, z, b, gs, dtype, f"M={M} K={K} gs={gs} split={w is not None}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("N,K,gs,M", [(4096, 896, 128, 17), (4112, 896, 896, 33), (9728, 896, 128, 64),
                                       (8208, 1024, 256, 47), (1152, 896, 128, 65), (1168, 1024, 1024, 128),
                                       (4480, 1024, 128, 17), (4112, 1024, 512, 33), (6160, 896, 128, 62),
