@@ -155,10 +155,12 @@ int ns_rope_reshape_and_cache(void* q_out, const void* query,
  * most 1024.
  * dtype is NS_DTYPE_F16 or NS_DTYPE_BF16.  N must be a multiple of 16, K and
  * group_size multiples of 32 with K a multiple of group_size; qweight 16-byte
- * aligned, out 8-byte aligned.  Up to 128 rows one kernel dequantises each
- * weight tile per 16 or 64 tokens; above, a tiled GEMM (K a multiple of 64,
- * no norm_weight, bias 8-byte and zeros 4-byte aligned; otherwise the first
- * kernel) dequantises it once per 128 or 256 tokens.
+ * aligned, out 8-byte aligned.  Up to 128 rows a register kernel dequantises
+ * each weight tile per 16 or 64 tokens, or (K and group_size multiples of 128,
+ * zeros 4-byte aligned, sizes where it is faster) a stream through LDS per 16 or
+ * 32; above, a tiled GEMM (K and group_size multiples of 64, no norm_weight, bias
+ * 8-byte and zeros 4-byte aligned; otherwise the register kernel) once per 64 or
+ * 128 tokens.  ns_int4_linear_kernel tells which.
  */
 int ns_int4_linear(void* out, const void* x, int64_t x_stride_row,
                    const void* qweight, const void* scales, const void* zeros, const void* bias,
@@ -173,18 +175,22 @@ int ns_int4_linear(void* out, const void* x, int64_t x_stride_row,
  * as ns_int4_linear; the fp32 partial sums of each split go to `workspace`
  * and the last split of a tile adds them in split order (deterministic) and
  * runs the epilogue.  Up to 128 tokens the split count (up to 8) depends on
- * how many workgroups the layer's tiles make; above (tiled
- * GEMM), the tiles of the last dispatch round split (all tiles when one round
- * holds them) when they fill at most half of the device's slots, within
- * those slots and with at least 8 K steps of 64 a split, so it depends on N,
- * K and the number of token tiles, and the partials never exceed one round
- * of fp32 tiles (32 MiB).
+ * how many workgroups the layer's tiles make.  Above (tiled GEMM), the tiles of
+ * the last dispatch round that lie past a whole round, or past one tile per
+ * CU (all of them when there are no more), split up to 4 ways where a model of
+ * the device's time finds that faster: at most 256 tiles, within the slots
+ * left in the round and with at least 8 K steps of 64 a split.  So it depends
+ * on N, K and the number of token tiles, and the partials never exceed one round of
+ * fp32 tiles (32 MiB).
  * Same replacement as ns_int4_linear (reference
  * nanoserve/quant.py:157-158).  workspace: 256-byte aligned,
  * ns_int4_linear_splitk_workspace_size(M, N, K) bytes, zeroed once before
  * first use; every call leaves its arrival counters at zero.  Calls that
  * overlap in time must not share a workspace.  Shapes that do not split
- * (size 0) ignore it.
+ * (size 0) ignore it.  Where the register kernel (up to 128 tokens; its rule
+ * counts also when another kernel takes the call) or the tiled GEMM splits, a
+ * missing, misaligned or smaller workspace is NS_ERR_INVALID_ARG; a call that
+ * only the weight stream would split runs unsplit without it.
  */
 size_t ns_int4_linear_splitk_workspace_size(int64_t M, int N, int K);
 int ns_int4_linear_splitk(void* out, const void* x, int64_t x_stride_row,
@@ -244,7 +250,7 @@ int ns_int4_linear_rope_cache(void* q_out, const void* x, int64_t x_stride_row,
  * the model-dtype weights of an INT4 layer: dequantize_int4 (reference
  * nanoserve/quant.py:83-95), bit for bit, in one pass.  For large token
  * counts a library GEMM on this weight is faster than ns_int4_linear, which
- * dequantises each weight tile once per 64-token tile.  K and group_size
+ * dequantises each weight tile once per 64- or 128-token tile.  K and group_size
  * multiples of 8, K a multiple of group_size.
  */
 int ns_int4_dequantize(void* out, const void* qweight, const void* scales, const void* zeros,

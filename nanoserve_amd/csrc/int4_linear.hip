@@ -749,7 +749,9 @@ hipError_t launch_int4_linear(const Int4LinearParams& p, hipStream_t stream, int
 // --------------------------------------------------------------------------
 
 // Eight codes -> weights in the order k = 0, 4, 1, 5, 2, 6, 3, 7, by the
-// arithmetic of dequant8_mix.  Nibbles e and e + 4 lie 16 bits apart, so one
+// arithmetic of dequant8_mix.  Both use the published magic-bias conversion (Kim et
+// al., "Who Says Elephants Can't Run", 2022): an integer or-ed into the mantissa of f16
+// 1024 reads as 1024 + it.  Nibbles e and e + 4 lie 16 bits apart, so one
 // and-or makes an f16 pair of them: 1024 + q for even e, 1024 + 16 q for odd
 // e (the nibble one position up), which one packed f16 add of -(1024 + z), or
 // one packed fma with 1/16 and -(64 + z), turns into q - z exactly.
@@ -1694,10 +1696,11 @@ constexpr int gemm_lds(int bm, int bn, int nst) {
 // graph-replayed): the pick is within 5% of the fastest in 792 of 800 and 14%
 // behind at worst (896 x 2048 at 1500 tokens, 22.6 / 19.7 us; 2048 x 2048 at 600,
 // 21.9 / 19.7).  Against shapes by thresholds on the tile count and splits of a
-// last round only, both measured: down_proj (896 x 4864) at 512 / 1500 / 4700 tokens 24.4 / 50.4 / 112 -> 20.5 / 31.4 / 73.7 us, 3584 x 14336 at
-// 200 / 800 / 1200 / 2000 tokens 74.7 / 176 / 313 / 366 -> 55.1 / 144 / 209 / 288
-// us, 28672 x 3584 at 200 / 300 tokens 106 / 150 -> 78.4 / 116 us, gate|up (9728 x
-// 896) at 700 tokens 35.1 -> 28.0 us; no call of the 800 is over 2.5% behind them.
+// last round only, both measured: down_proj (896 x 4864) at 512 / 1500 / 4700
+// tokens 24.4 / 50.4 / 112 -> 20.5 / 31.4 / 73.7 us, 3584 x 14336 at 200 / 800 /
+// 1200 / 2000 tokens 74.7 / 176 / 313 / 366 -> 55.1 / 144 / 209 / 288 us, 28672 x
+// 3584 at 200 / 300 tokens 106 / 150 -> 78.4 / 116 us, gate|up (9728 x 896) at 700
+// tokens 35.1 -> 28.0 us; no call of the 800 is over 2.5% behind them.
 //
 // From 512 tiles of 128 x 128 those are taken outright, so the choice and its
 // partials repeat with every 512 token tiles.  (They mostly win there, but not past
@@ -1798,7 +1801,8 @@ namespace {
 
 // Split-K workspace: a fixed region of u32 arrival counters (one per tile,
 // zero between calls), then the partial sums.  The region has the same size
-// for every M: the fused kernel only splits when 2 * tiles <= 256 and the
+// for every M: the register kernel only splits when 2 * tiles <= 256, the weight
+// stream when its workgroups are fewer than 256, and the
 // GEMM splits at most gemm::kMaxSplitTiles tiles, so at most 256 counters exist,
 // and the partials of any call start past every counter any other call may
 // use.  One workspace can therefore serve calls of every token count in turn
@@ -1812,8 +1816,8 @@ struct SplitkLayout {
 };
 
 // Token counts above kGemmMinRows take the GEMM (when K is a whole number of
-// its steps), the rest the fused kernel with 16 bytes of partials per lane,
-// tile and split.
+// its steps), the rest the weight stream (`stream`) or the register kernel, both
+// with 16 bytes of partials per lane, tile and split.
 SplitkLayout splitk_layout(int64_t M, int N, int K, bool stream) {
   SplitkLayout l{1, 0, 0};
   if (M <= 0) return l;

@@ -826,13 +826,15 @@ __global__ __launch_bounds__(W * 64) void paged_decode_kernel(AttnParams p) {
 // columns a wave) halves the chain of steps and makes the most workgroups; the
 // wide one (384 columns at D = 64, 256 at D = 128, eight waves side by side)
 // loads each K/V tile for three / two times as many columns, and its waves
-// share one tile instead of two.  What bounds both is the vector ALU's issue
-// slots (SQ counters, 2048 rows x 7 heads behind 9392 keys, D = 64: 180 VALU
-// operations, 32 exponentials of four slots and 36 MFMAs per wave and 64 keys
-// x 32 columns, 1376 of about 1620 cycles in the wide kernel; 228 before the
-// operand reads took constant offsets and the table look-ups moved off the
-// loads' path) plus the barriers.  The host takes the wide one where it makes
-// enough workgroups (prefill_wide).
+// share one tile instead of two.  The wide one is bound by the vector ALU's issue
+// slots and its barriers (SQ counters, 2048 rows x 7 heads behind 9392 keys, D = 64:
+// 180 VALU operations, 32 exponentials of four slots and 36 MFMAs per wave and 64
+// keys x 32 columns, 1376 of about 1620 cycles; 228 before the operand reads took
+// constant offsets and the table look-ups moved off the loads' path).  The narrow
+// one, on the same batch (224 workgroups), issues VALU in 56% of its
+// waves' cycles, two to a SIMD, and has the matrix cores busy in 30%; its waves
+// wait for barriers and loads in 35%, and 32 CUs hold no workgroup.  The host takes
+// the wide one where it is the faster (prefill_wide).
 //
 // LDS layout of a slot: K tile then V tile, both [KT][D] rows of 16-byte
 // chunks, chunk c of key k stored at chunk c ^ k_swz(k) (K) or c ^ pf_v_swz(k)
